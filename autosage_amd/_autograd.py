@@ -7,7 +7,7 @@ backward formulas built from the same native kernels:
 * ``Y = A·X`` (A: CSR, weights ``val`` or ones):
   ``dX = Aᵀ·dY`` — a native SpMM over the transposed CSR — and
   ``dval[e] = <dY[row(e)], X[col(e)]>`` — a native SDDMM;
-  both on the degree-split schedules (same bits as the whole-graph kernels);
+  the SpMM on the schedule that suits the graph (same bits on each);
   the column-sliced operators take dX on the column-sliced SpMM instead
   (same fp64-partial contract as their forward).
   With bf16 / fp16 features both come from the rounded 16-bit kernels
@@ -57,12 +57,11 @@ def _build_transpose(crow: torch.Tensor, col: torch.Tensor) -> tuple[torch.Tenso
     return crow_t, rows.index_select(0, perm).contiguous(), perm
 
 
-# The backward products run on the degree-split schedules when the graph has
-# hub rows: bit-identical to the whole-graph kernels (the SpMM keeps CSR
-# order per output, the SDDMM the reference's dot order), but hub rows are
-# split across waves, which matters on skewed graphs (one wave per 200k-edge
-# row is several times slower).  Without hub rows the whole-graph SpMM runs
-# (memoised per-graph row count, one launch).
+# The backward SpMMs run on the degree-split schedule when the graph has hub
+# rows: bit-identical to the whole-graph kernel (CSR order per output), but
+# hub rows are split across waves, which matters on skewed graphs (one wave
+# per 200k-edge row is several times slower).  Without hub rows the
+# whole-graph SpMM runs (memoised per-graph row count, one launch).
 _HUB_THRESHOLD = 1024
 
 
@@ -104,7 +103,7 @@ def _column_slices_allowed() -> bool:
 
 
 def _sddmm(crow, col, query, key):
-    return torch.ops.autosage.sddmm_csr_split(crow, col, query, key, 4, _HUB_THRESHOLD)
+    return torch.ops.autosage.sddmm_csr(crow, col, query, key)
 
 
 def _spmm_setup(ctx, inputs, output) -> None:

@@ -29,7 +29,7 @@ from . import _env
 from ._memo import GraphMemo
 
 LIBRARY_NAME = "libautosage_hip.so"
-ABI_VERSION = 9
+ABI_VERSION = 10
 HUB_EXACT = 0
 HUB_SPLIT64 = 1
 # 16-bit feature types of as_spmm_csr_rounded_16 (AS_DTYPE_BF16 / AS_DTYPE_F16)
@@ -75,6 +75,8 @@ _SIGNATURES = {
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_int, _c_int,
          _c_ptr],
     ),
+    "as_sddmm_csr_edges_f32": (
+        _c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr]),
     "as_sddmm_csr_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr]),
     "as_sddmm_split_workspace_bytes": (_c_size, [_c_i64]),
     "as_sddmm_csr_split_f32": (
@@ -710,20 +712,23 @@ def spmm_rounded_16_impl(crow, col, val, x, column_slices: bool):
 # the 124M-edge attention graph, 11 % on the skewed 115M-edge graph.
 
 
-# fp32 sddmm_csr: every output keeps the reference kernel's dot order on any
-# schedule, so graphs that can hold a row of this many edges take the split
-# schedule (such rows cut into 2048-edge chunks over a workgroup's waves)
-# instead of one wave per row; the bits are the same.
-SDDMM_HUB_THRESHOLD = 1024
-SDDMM_WAVES = 4
+def _sddmm_edges_f32(crow, col, query, key, out) -> None:
+    """fp32 SDDMM over blocks of 64 edges in CSR order (any widths, any row
+    lengths; ``key`` may have more rows than ``query``): one launch, no
+    workspace, the reference kernel's dot order."""
+    n, f = query.shape
+    with _on(query.device):
+        status = library().as_sddmm_csr_edges_f32(
+            _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, key.size(0), col.numel(), f,
+            _stream(query.device)
+        )
+    _raise(status, "autosage::sddmm_csr")
 
 
 def sddmm_csr_impl(crow, col, query, key):
     check_sddmm_inputs(crow, col, query, key, allow_16=True)
     if query.dtype in DTYPES_16:
         return sddmm_edges_16_impl(crow, col, query, key)
-    if col.numel() >= SDDMM_HUB_THRESHOLD:
-        return sddmm_csr_split_impl(crow, col, query, key, SDDMM_WAVES, SDDMM_HUB_THRESHOLD)
     _maybe_validate(crow, col)
     nnz = col.numel()
     n, f = query.shape
@@ -732,11 +737,7 @@ def sddmm_csr_impl(crow, col, query, key):
     out = torch.empty(nnz, dtype=query.dtype, device=query.device)
     if n == 0 or nnz == 0:
         return out
-    with _on(query.device):
-        status = library().as_sddmm_csr_f32(
-            _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, nnz, f, _stream(query.device)
-        )
-    _raise(status, "autosage::sddmm_csr")
+    _sddmm_edges_f32(crow, col, query, key, out)
     return out
 
 
@@ -754,14 +755,8 @@ def sddmm_csr_split_impl(crow, col, query, key, warps_per_block, hub_threshold):
     out = torch.empty(nnz, dtype=query.dtype, device=query.device)
     if n == 0 or nnz == 0:
         return out
-    lib = library()
-    ws = _workspace(lib.as_sddmm_split_workspace_bytes(n), query.device)
-    with _on(query.device):
-        status = lib.as_sddmm_csr_split_f32(
-            _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, nnz, f, int(warps_per_block),
-            int(hub_threshold), _ptr(ws), ws.numel(), _stream(query.device),
-        )
-    _raise(status, "autosage::sddmm_csr_split")
+    # fp32: every schedule gives the same bits, and the blocks of edges need none
+    _sddmm_edges_f32(crow, col, query, key, out)
     return out
 
 
@@ -1025,16 +1020,9 @@ def sddmm_csr_rect_impl(crow, col, query, key):
                 _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, key.size(0), nnz, f,
                 DTYPES_16[query.dtype], _ptr(ws), ws.numel(), _stream(query.device),
             )
-        elif nnz >= SDDMM_HUB_THRESHOLD:
-            # fp32 kernels address the key through the column indices only
-            ws = _workspace(lib.as_sddmm_split_workspace_bytes(n), query.device)
-            status = lib.as_sddmm_csr_split_f32(
-                _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, nnz, f, SDDMM_WAVES,
-                SDDMM_HUB_THRESHOLD, _ptr(ws), ws.numel(), _stream(query.device),
-            )
         else:
-            status = lib.as_sddmm_csr_f32(_ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, nnz, f,
-                                          _stream(query.device))
+            status = lib.as_sddmm_csr_edges_f32(_ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n,
+                                                key.size(0), nnz, f, _stream(query.device))
     _raise(status, "autosage row-shard SDDMM")
     return out
 

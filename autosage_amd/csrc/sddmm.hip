@@ -6,14 +6,9 @@
 // Summation order (both reference kernels, :12-17 and :39-49): the 32 lanes
 // of a warp each keep one fp32 partial, lane l adding features l, l+32,
 // l+64, ... with fma; the 32 partials are then combined by the 16/8/4/2/1
-// shfl_down tree.  Every kernel here reproduces exactly that order, so all
-// SDDMM entry points give identical bits.
-//
-// gfx950 mapping: G lanes of a wave64 work on one edge and each lane holds
-// S = 32/G of the 32 partials (partial l = S·j + s in lane j, slot s), loaded
-// as one S-wide vector per 32-feature block.  64/G edges are in flight per
-// wave iteration.  Tree steps with offset o >= S are lane butterflies
-// (xor o/S, inside the G-lane group); steps with o < S add slots in-lane.
+// shfl_down tree.  The fp32 kernel reproduces exactly that order, so all
+// fp32 SDDMM entry points give identical bits; the 16-bit kernels follow
+// their own rule (below).
 #include "as_device.h"
 #include "as_internal.h"
 #include "elem16.h"
@@ -26,123 +21,8 @@ namespace {
 
 constexpr int kChunkEdges = 2048;  // edges per hub work item
 
-template <int S>
-__device__ __forceinline__ float ref_tree(float (&p)[S]) {
-#pragma unroll
-  for (int o = 16; o >= S; o >>= 1) {
-#pragma unroll
-    for (int s = 0; s < S; ++s) p[s] += __shfl_xor(p[s], o / S, 64);
-  }
-#pragma unroll
-  for (int o = S / 2; o >= 1; o >>= 1) {
-#pragma unroll
-    for (int s = 0; s < o; ++s) p[s] += p[s + o];
-  }
-  return p[0];
-}
-
-// Dot products of one query row against UE·NG key rows (vector path,
-// F = 32·MF features, G lanes per edge).  Writes out[e] for valid edges.
-template <int G, int MF, int UE>
-__device__ __forceinline__ void dot_edges_vec(const int64_t* __restrict__ col, const float* __restrict__ key,
-                                              float* __restrict__ out, int64_t F, const float (&qv)[MF][32 / G],
-                                              int64_t first, int64_t stride, int64_t end, int g, int j) {
-  constexpr int S = 32 / G;
-  FVec<S> kv[UE][MF];
-  bool ok[UE];
-  int64_t e[UE];
-#pragma unroll
-  for (int u = 0; u < UE; ++u) {
-    e[u] = first + u * stride + g;
-    ok[u] = e[u] < end;
-    const int64_t ee = ok[u] ? e[u] : end - 1;
-    const int c = static_cast<int>(col[ee]);
-    const float* kr = key + row_offset(c, F) + S * j;
-#pragma unroll
-    for (int m = 0; m < MF; ++m) kv[u][m] = load_vec<S>(kr + 32 * m);
-  }
-#pragma unroll
-  for (int u = 0; u < UE; ++u) {
-    float p[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) p[s] = 0.f;
-#pragma unroll
-    for (int m = 0; m < MF; ++m) {
-#pragma unroll
-      for (int s = 0; s < S; ++s) p[s] = __builtin_fmaf(qv[m][s], kv[u][m].v[s], p[s]);
-    }
-    const float d = ref_tree<S>(p);
-    if (ok[u] && j == 0) out[e[u]] = d;
-  }
-}
-
-// Scalar path for any F: 32 lanes per edge (exactly the reference lane
-// mapping), two edges per wave iteration; the query row is re-read from cache.
-__device__ __forceinline__ void dot_edges_scalar(const int64_t* __restrict__ col, const float* __restrict__ qrow,
-                                                 const float* __restrict__ key, float* __restrict__ out, int64_t F,
-                                                 int64_t first, int64_t stride, int64_t end, int g, int j) {
-  const int64_t e = first + g;
-  const bool ok = e < end;
-  const int64_t ee = ok ? e : end - 1;
-  const int c = static_cast<int>(col[ee]);
-  const float* kr = key + row_offset(c, F);
-  float p[1] = {0.f};
-  for (int64_t f = j; f < F; f += 32) p[0] = __builtin_fmaf(qrow[f], kr[f], p[0]);
-  const float d = ref_tree<1>(p);
-  if (ok && j == 0) out[e] = d;
-  (void)stride;
-}
-
-template <int G, int MF>
-__device__ __forceinline__ void load_query(const float* __restrict__ qrow, int j, float (&qv)[MF][32 / G]) {
-  constexpr int S = 32 / G;
-#pragma unroll
-  for (int m = 0; m < MF; ++m) {
-    const FVec<S> t = load_vec<S>(qrow + 32 * m + S * j);
-#pragma unroll
-    for (int s = 0; s < S; ++s) qv[m][s] = t.v[s];
-  }
-}
-
-// One wave computes every edge of `row` (vector or scalar path).
-template <int G, int MF, bool VEC>
-__device__ __forceinline__ void sddmm_row(const int64_t* __restrict__ col, const float* __restrict__ query,
-                                          const float* __restrict__ key, float* __restrict__ out, int64_t F,
-                                          int64_t row, int64_t rs, int64_t re) {
-  const int lane = lane_id();
-  const int g = lane / G;
-  const int j = lane % G;
-  if constexpr (VEC) {
-    constexpr int NG = kWave / G;
-    constexpr int UE = MF <= 2 ? 4 : 2;
-    float qv[MF][32 / G];
-    load_query<G, MF>(query + row * F, j, qv);
-    for (int64_t base = rs; base < re; base += NG * UE) dot_edges_vec<G, MF, UE>(col, key, out, F, qv, base, NG, re, g, j);
-  } else {
-    const float* qrow = query + row * F;
-    for (int64_t base = rs; base < re; base += 2) dot_edges_scalar(col, qrow, key, out, F, base, 2, re, g, j);
-  }
-}
-
-// One wave per row; rows of degree >= hub_threshold are left to the hub
-// kernel (csrc/sddmm_csr_op.cu:35-37).
-template <int G, int MF, bool VEC>
-__global__ __launch_bounds__(kBlock) void sddmm_rows_kernel(const int64_t* __restrict__ crow,
-                                                            const int64_t* __restrict__ col,
-                                                            const float* __restrict__ query,
-                                                            const float* __restrict__ key, float* __restrict__ out,
-                                                            int64_t n, int64_t F, int64_t hub_threshold,
-                                                            int64_t idx_base) {
-  const int64_t row = idx_base + static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
-  if (row >= n) return;
-  const int64_t rs = uniform_i64(crow[row]);
-  const int64_t re = uniform_i64(crow[row + 1]);
-  if (re - rs >= hub_threshold || re == rs) return;
-  sddmm_row<G, MF, VEC>(col, query, key, out, F, row, rs, re);
-}
-
-// Work items of the hub kernel: hub h (order[h], h < counts[0]) is cut into
-// ceil(deg / kChunkEdges) chunks; chunk_off[h] is the exclusive prefix and
+// Work items of the 16-bit split schedule: hub h (order[h],
+// h < counts[0]) is cut into ceil(deg / kChunkEdges) chunks; chunk_off[h] is the exclusive prefix and
 // counts[2] the total.  One workgroup of 1024 threads.
 __global__ __launch_bounds__(1024) void hub_chunk_scan_kernel(const int64_t* __restrict__ crow,
                                                               const int32_t* __restrict__ order,
@@ -179,58 +59,281 @@ __global__ __launch_bounds__(1024) void hub_chunk_scan_kernel(const int64_t* __r
   if (threadIdx.x == 0) counts[2] = total;
 }
 
-// Split SDDMM in one launch.  Workgroups [0, hub_blocks) stride over the hub
-// chunk items (2048-edge pieces of hub rows; usually one each); the rest take
-// the light rows in row order, one per wave, skipping hub and empty rows.
-// Hub workgroups have the lowest indices, so they are dispatched first.
-template <int G, int MF, bool VEC>
-__global__ __launch_bounds__(512) void sddmm_scheduled_kernel(
-    const int64_t* __restrict__ crow, const int64_t* __restrict__ col, const float* __restrict__ query,
-    const float* __restrict__ key, float* __restrict__ out, int64_t n, int64_t F, int64_t hub_threshold,
-    const int32_t* __restrict__ order, const int32_t* __restrict__ counts, const int32_t* __restrict__ chunk_off,
-    int64_t hub_blocks, int64_t block_base) {
-  constexpr int NG = VEC ? kWave / G : 2;
+// Lane i: the row of edge b + min(i, cnt - 1), given r, the row of edge b.
+// Every lane of the wave must be active.  The rounds end at the last row
+// whatever crow holds, and the result is clamped to [0, n).
+__device__ __forceinline__ int block_edge_rows(const int64_t* __restrict__ crow, int64_t n, int64_t b, int cnt,
+                                               int64_t r) {
   const int lane = lane_id();
-  const int g = lane / (VEC ? G : 32);
-  const int j = lane % (VEC ? G : 32);
-  const int wave = wave_in_block();
-  const int waves = static_cast<int>(blockDim.x >> 6);
-  const int64_t block = block_base + blockIdx.x;
-  if (block < hub_blocks) {
-    const int64_t hubs = counts[0];
-    const int64_t items = counts[2];
-    for (int64_t item = block; item < items; item += hub_blocks) {
-      int64_t lo = 0;
-      int64_t hi = hubs - 1;
-      while (lo < hi) {
-        const int64_t mid = (lo + hi + 1) >> 1;
-        if (chunk_off[mid] <= item) lo = mid;
-        else hi = mid - 1;
-      }
-      const int64_t row = uniform_i64(order[lo]);
-      const int64_t rs = uniform_i64(crow[row]);
-      const int64_t re = uniform_i64(crow[row + 1]);
-      const int64_t cs = rs + (item - uniform_i64(chunk_off[lo])) * kChunkEdges;
-      const int64_t ce = cs + kChunkEdges < re ? cs + kChunkEdges : re;
-      if constexpr (VEC) {
-        float qv[MF][32 / G];
-        load_query<G, MF>(query + row * F, j, qv);
-        for (int64_t base = cs + static_cast<int64_t>(wave) * NG; base < ce; base += static_cast<int64_t>(waves) * NG)
-          dot_edges_vec<G, MF, 1>(col, key, out, F, qv, base, NG, ce, g, j);
-      } else {
-        const float* qrow = query + row * F;
-        for (int64_t base = cs + static_cast<int64_t>(wave) * 2; base < ce; base += static_cast<int64_t>(waves) * 2)
-          dot_edges_scalar(col, qrow, key, out, F, base, 2, ce, g, j);
+  const int i = lane < cnt ? lane : cnt - 1;
+  int row = -1;
+  for (int64_t rr = r;; rr += kWave) {
+    // rel: where row rr + lane ends (row n - 1 for lanes past it), relative
+    // to b, clamped to [0, 64]
+    const int64_t left = n - 1 - rr;  // >= 0
+    const int lim = left < kWave ? static_cast<int>(left) : kWave;
+    const int64_t d = crow[rr + 1 + (lane < lim ? lane : lim)] - b;
+    const int rel = d < 0 ? 0 : (d > kWave ? kWave : static_cast<int>(d));
+    // pos = #{l : rel_l <= i}, the ends being non-decreasing in l
+    int pos = 0;
+#pragma unroll
+    for (int s = kWave / 2; s >= 1; s >>= 1) {
+      const int v = __builtin_amdgcn_ds_bpermute((pos + s - 1) * 4, rel);
+      pos = v <= i ? pos + s : pos;
+    }
+    const int rel_last = __builtin_amdgcn_readlane(rel, kWave - 1);
+    if (pos == kWave - 1 && rel_last <= i) pos = kWave;
+    if (row < 0 && pos < kWave) row = static_cast<int>(rr + pos);
+    if (rel_last >= cnt || rr + kWave >= n) break;
+  }
+  const int last = static_cast<int>(n - 1);
+  return row < 0 || row > last ? last : row;
+}
+
+// The row holding edge e: the last r < n with crow[r] <= e (0 if none), by
+// the whole wave, 64 probes a step; ends after log64(n) steps whatever crow
+// holds.
+__device__ __forceinline__ int64_t wave_row_of_edge(const int64_t* __restrict__ crow, int64_t n, int64_t e) {
+  int64_t lo = 0;
+  int64_t hi = n;
+  while (hi - lo > 1) {
+    const int64_t step = (hi - lo + kWave - 1) / kWave;
+    const int64_t probe = lo + lane_id() * step;
+    const uint64_t below = __ballot(probe < hi && crow[probe] <= e);
+    if (below != 0) lo += static_cast<int64_t>(63 - __builtin_clzll(below)) * step;
+    hi = lo + step < hi ? lo + step : hi;
+  }
+  return lo;
+}
+
+// ---- fp32 SDDMM by blocks of edges ------------------------------------------
+// The edges in CSR order, 64 a block, whatever the rows; every output keeps
+// the reference's order (file comment).  8 lanes per edge and 8 edges per
+// lane group: lane j of group g holds partials 4j .. 4j+3 of edges 8g .. 8g+7,
+// one 16-byte key load (and query load) per 32 features and edge, so every
+// gather instruction carries 8 edges however short the rows are.  Loads are
+// aligned to 4 bytes only, so any F >= 4 takes vector lanes: the last partial
+// block reads at F - 4 and shifts.
+// The tree's three lane steps halve the edges a lane keeps (8, 4, 2, 1): the
+// lane with the step's bit set keeps the upper half and receives its partner's
+// part of it, 28 lane exchanges for 64 edges where a butterfly per edge takes
+// 96, and lane i ends with edge i (one coalesced store).
+//
+// What bounds it: the gathers, at the memory's rate where K is beyond the
+// caches (1M rows, 16.8M edges, F = 64: 0.655 ms, 6.6 TB/s of gathered bytes),
+// at the L2's where it is not.  Against one wave per row and the split
+// schedule (us): 100k rows, 1.2M edges, F = 47 446 -> 34, F = 64 125 -> 30, F = 100
+// 690 -> 52 (F % 32 != 0 used to take 4-byte lanes and 2 edges an instruction);
+// 1M rows, 50M edges, hubs of 200k edges, F = 64 1508 -> 809, F = 100 7370 -> 1535.
+//
+// How a row's 32-feature blocks are taken.  F % 32 == 0: one block of all 8
+// edges at a time (each a whole 128-byte line of X).  Otherwise rows start
+// inside lines and neighbouring blocks share one, so an edge's blocks (up to 4)
+// are read together before the next edge's; taken one at a time the shared
+// lines were fetched twice (F = 100, 1M rows: 1.63 ms, 2 blocks of 2 edges at a
+// time 1.44, 4 blocks of 2 edges 1.46, 4 blocks of 1 edge 1.24).
+typedef float Float4U __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool OFF32>
+struct RowOff;
+template <>
+struct RowOff<true> {
+  uint32_t v;
+};
+template <>
+struct RowOff<false> {
+  int64_t v;
+};
+template <bool OFF32>
+__device__ __forceinline__ RowOff<OFF32> row_off(int row, uint32_t row_bytes, uint32_t lane_off) {
+  if constexpr (OFF32) return {static_cast<uint32_t>(row) * row_bytes + lane_off};
+  else return {static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(row)) * row_bytes + lane_off)};
+}
+template <bool OFF32>
+__device__ __forceinline__ Float4U load4(const char* __restrict__ base, RowOff<OFF32> off, int delta) {
+  if constexpr (OFF32) return *reinterpret_cast<const Float4U*>(base + (off.v + static_cast<uint32_t>(delta)));
+  else return *reinterpret_cast<const Float4U*>(base + (off.v + delta));
+}
+
+__device__ __forceinline__ Float4U shifted(Float4U v, int shift) {
+  if (shift & 1) v = Float4U{v.y, v.z, v.w, v.w};
+  if (shift & 2) v = Float4U{v.z, v.w, v.w, v.w};
+  return v;
+}
+
+__device__ __forceinline__ float lane_xor4(float v) {
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (4 << 10) | 0x1f));
+}
+__device__ __forceinline__ float lane_xor2(float v) {  // quad_perm [2,3,0,1]
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4e, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_xor1(float v) {  // quad_perm [1,0,3,2]
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));
+}
+
+// Adds 32-feature blocks [m0, m0 + MB) of the 8 edges to p, UE edges at a
+// time.  Block m of lane j holds features 32m + 4j ..; the row's last block
+// (MASK) reads at F - 4 where that passes F.  TAIL: 0 F % 32 == 0, 1 whole
+// vectors (4 | F), 2 shifted vectors (F >= 4), 3 elements (F < 4).
+template <int MB, int TAIL, bool MASK, bool OFF32, bool ONE>
+__device__ __forceinline__ void edge_blocks_dots(const char* __restrict__ kb, const char* __restrict__ qb, int F,
+                                                 int m0, const RowOff<OFF32> (&ko)[8],
+                                                 const RowOff<OFF32> (&qo)[ONE ? 1 : 8], float (&p)[8][4]) {
+  constexpr int UE = MB == 1 ? 8 : (MB == 2 ? 2 : 1);
+  const int j4 = 4 * (lane_id() & 7);
+  int delta[MB], shift[MB], left[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const int start = 32 * (m0 + m) + j4;
+    delta[m] = (m0 + m) * 128;
+    left[m] = F - start;
+    shift[m] = 0;
+    if (TAIL == 1 || TAIL == 2) {
+      if (MASK && m == MB - 1) {
+        const int from = start < F - 4 ? start : F - 4;
+        delta[m] = (from - j4) * 4;
+        shift[m] = start - from;  // used where left > 0, then <= 3
       }
     }
-    return;
   }
-  const int64_t row = (block - hub_blocks) * waves + wave;
-  if (row >= n) return;
-  const int64_t rs = uniform_i64(crow[row]);
-  const int64_t re = uniform_i64(crow[row + 1]);
-  if (re - rs >= hub_threshold || re == rs) return;
-  sddmm_row<G, MF, VEC>(col, query, key, out, F, row, rs, re);
+#pragma unroll
+  for (int h = 0; h < 8; h += UE) {
+    Float4U k[UE][MB];
+    Float4U q[ONE ? 1 : UE][MB];
+#pragma unroll
+    for (int u = 0; u < UE; ++u) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        if constexpr (TAIL == 3) {
+          k[u][m] = Float4U{0.f, 0.f, 0.f, 0.f};
+          if (!ONE || u == 0) q[ONE ? 0 : u][m] = Float4U{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int s = 0; s < 3; ++s) {
+            if (s < left[m]) {
+              k[u][m][s] = *reinterpret_cast<const float*>(kb + ko[h + u].v + 4 * s);
+              if (!ONE || u == 0)
+                q[ONE ? 0 : u][m][s] = *reinterpret_cast<const float*>(qb + qo[ONE ? 0 : h + u].v + 4 * s);
+            }
+          }
+        } else {
+          k[u][m] = load4<OFF32>(kb, ko[h + u], delta[m]);
+          if (!ONE || u == 0) q[ONE ? 0 : u][m] = load4<OFF32>(qb, qo[ONE ? 0 : h + u], delta[m]);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < UE; ++u) {
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        const bool masked = TAIL != 0 && MASK && m == MB - 1;
+        Float4U kk = k[u][m];
+        Float4U qq = q[ONE ? 0 : u][m];
+        if (TAIL == 2 && masked) {
+          kk = shifted(kk, shift[m]);
+          qq = shifted(qq, shift[m]);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const float t = __builtin_fmaf(qq[s], kk[s], p[h + u][s]);
+          // a skipped feature leaves the sum as it is (0 * k would not, for
+          // an infinite k or a sum of -0)
+          p[h + u][s] = !masked || (TAIL == 1 ? 0 : s) < left[m] ? t : p[h + u][s];
+        }
+      }
+    }
+    if constexpr (UE < 8) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// One block of 64 edges: the dot product of edge `lane`.  my_c / my_row: lane
+// i holds the column / row of edge i.  ONE: every edge is in row my_row.
+// F's 32-feature blocks are taken CB at a time, the last LAST together.
+template <int CB, int LAST, int TAIL, bool OFF32, bool ONE>
+__device__ __forceinline__ float edge_block_dots(const char* __restrict__ kb, const char* __restrict__ qb, int F,
+                                                 int my_c, int my_row) {
+  const int lane = lane_id();
+  const uint32_t row_bytes = static_cast<uint32_t>(F) * 4u;
+  const uint32_t lane_off = static_cast<uint32_t>((lane & 7) * 16);
+  RowOff<OFF32> ko[8];
+  RowOff<OFF32> qo[ONE ? 1 : 8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int addr = ((lane & 56) + u) * 4;
+    ko[u] = row_off<OFF32>(__builtin_amdgcn_ds_bpermute(addr, my_c), row_bytes, lane_off);
+    if constexpr (!ONE) qo[u] = row_off<OFF32>(__builtin_amdgcn_ds_bpermute(addr, my_row), row_bytes, lane_off);
+  }
+  if constexpr (ONE) qo[0] = row_off<OFF32>(my_row, row_bytes, lane_off);
+  float p[8][4];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) p[u][s] = 0.f;
+  }
+  const int last = (F + 31) / 32 - LAST;
+  if constexpr (CB > 0) {
+    for (int m = 0; m < last; m += CB) edge_blocks_dots<CB, TAIL, false, OFF32, ONE>(kb, qb, F, m, ko, qo, p);
+  }
+  edge_blocks_dots<LAST, TAIL, TAIL != 0, OFF32, ONE>(kb, qb, F, CB > 0 ? last : 0, ko, qo, p);
+  const bool b4 = (lane & 4) != 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float keep = b4 ? p[u + 4][s] : p[u][s];
+      const float send = b4 ? p[u][s] : p[u + 4][s];
+      p[u][s] = keep + lane_xor4(send);
+    }
+  }
+  const bool b2 = (lane & 2) != 0;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float keep = b2 ? p[u + 2][s] : p[u][s];
+      const float send = b2 ? p[u][s] : p[u + 2][s];
+      p[u][s] = keep + lane_xor2(send);
+    }
+  }
+  const bool b1 = (lane & 1) != 0;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const float keep = b1 ? p[1][s] : p[0][s];
+    const float send = b1 ? p[0][s] : p[1][s];
+    p[0][s] = keep + lane_xor1(send);
+  }
+  return (p[0][0] + p[0][2]) + (p[0][1] + p[0][3]);
+}
+
+constexpr int kEdgeWaves = 4;  // waves per workgroup
+
+template <int CB, int LAST, int TAIL, bool OFF32>
+__global__ __launch_bounds__(kEdgeWaves * kWave) __attribute__((amdgpu_waves_per_eu(4))) void sddmm_edges_kernel(
+    const int64_t* __restrict__ crow, const int64_t* __restrict__ col, const float* __restrict__ query,
+    const float* __restrict__ key, float* __restrict__ out, int64_t n, int64_t nnz, int F, int64_t per_wave,
+    int64_t wave_base) {
+  const int64_t w = wave_base + static_cast<int64_t>(blockIdx.x) * kEdgeWaves + wave_in_block();
+  const int64_t b0 = uniform_i64(w * per_wave);
+  if (b0 >= nnz) return;  // wave-uniform
+  const int lane = lane_id();
+  const int64_t b1 = uniform_i64(b0 + per_wave < nnz ? b0 + per_wave : nnz);
+  const char* __restrict__ kb = reinterpret_cast<const char*>(key);
+  const char* __restrict__ qb = reinterpret_cast<const char*>(query);
+  int next_c = b0 + lane < b1 ? static_cast<int>(col[b0 + lane]) : 0;
+  int64_t r = uniform_i64(wave_row_of_edge(crow, n, b0));
+  for (int64_t b = b0; b < b1; b += kWave) {
+    const int cnt = b1 - b < kWave ? static_cast<int>(b1 - b) : kWave;
+    const int my_c = next_c;
+    if (b + kWave < b1) next_c = b + kWave + lane < b1 ? static_cast<int>(col[b + kWave + lane]) : 0;
+    float d;
+    if (uniform_i64(crow[r + 1]) >= b + cnt) {  // every edge of the block is in row r
+      d = edge_block_dots<CB, LAST, TAIL, OFF32, true>(kb, qb, F, my_c, static_cast<int>(r));
+    } else {
+      const int my_row = block_edge_rows(crow, n, b, cnt, r);
+      r = __builtin_amdgcn_readlane(my_row, cnt - 1);
+      d = edge_block_dots<CB, LAST, TAIL, OFF32, false>(kb, qb, F, my_c, my_row);
+    }
+    if (lane < cnt) out[b + lane] = d;
+  }
 }
 
 struct SddmmArgs {
@@ -243,38 +346,60 @@ struct SddmmArgs {
   int64_t f;
 };
 
-bool vec_ok(const SddmmArgs& a) {
-  const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) % 16) == 0; };
-  return a.f % 32 == 0 && a.f / 32 <= 8 && a.f > 0 && al(a.q) && al(a.k);
-}
+// Blocks of 64 edges a wave: 4 spread the row search and the start of the
+// chain over 256 edges (1M rows, 50M edges, F = 64 us at 1 / 2 / 4 / 8 blocks:
+// 1106 / 909 / 811 / 764), except that wide rows of a few edges, whose gathers run
+// at the memory's rate anyway, are better off in launch order (1M rows, 16.8M
+// edges: F = 96 924 / 951 / 963, F = 128 1229 / 1246 / 1259 at 1 / 2 / 4).
+// Fewer than 4 where that would leave fewer than 16,384 waves.
+constexpr int64_t kMaxEdgeBlocks = 4;
+constexpr int64_t kFillWaves = 16384;
+constexpr int64_t kShortRowDegree = 32;
+constexpr int64_t kWideRow = 96;
 
-int launch_sddmm_rows(const SddmmArgs& a, int64_t hub_threshold, hipStream_t stream) {
-  const int64_t blocks = (a.n + kWavesPerBlock - 1) / kWavesPerBlock;
-  const bool vec = vec_ok(a);
-  const int mf = static_cast<int>(a.f / 32);
+// n_keys: rows of the key, or -1 where the caller does not know them (64-bit
+// offsets then).
+void launch_sddmm_edges(const SddmmArgs& a, int64_t nnz, int64_t n_keys, hipStream_t s) {
+  int64_t per = nnz / (kFillWaves * kWave);
+  const bool in_order = a.f >= kWideRow && nnz < kShortRowDegree * a.n;
+  per = per < 1 || in_order ? 1 : (per > kMaxEdgeBlocks ? kMaxEdgeBlocks : per);
+  const int64_t per_wave = per * kWave;
+  const int64_t waves = (nnz + per_wave - 1) / per_wave;
+  const int64_t blocks = (waves + kEdgeWaves - 1) / kEdgeWaves;
+  const int64_t rows = a.n > n_keys ? a.n : n_keys;
+  const bool off32 = n_keys > 0 && rows * a.f * 4 <= (int64_t(1) << 32);
   for (int64_t b0 = 0; b0 < blocks; b0 += kMaxBlocksPerLaunch) {
     const int64_t nb = blocks - b0 < kMaxBlocksPerLaunch ? blocks - b0 : kMaxBlocksPerLaunch;
+#define AS_E32(CB, LAST, TAIL)                                                                                    \
+  do {                                                                                                          \
+    if (off32)                                                                                                  \
+      hipLaunchKernelGGL((sddmm_edges_kernel<CB, LAST, TAIL, true>), grid, dim3(kEdgeWaves * kWave), 0, s, a.crow, \
+                         a.col, a.q, a.k, a.out, a.n, nnz, static_cast<int>(a.f), per_wave, b0 * kEdgeWaves);   \
+    else                                                                                                        \
+      hipLaunchKernelGGL((sddmm_edges_kernel<CB, LAST, TAIL, false>), grid, dim3(kEdgeWaves * kWave), 0, s,     \
+                         a.crow, a.col, a.q, a.k, a.out, a.n, nnz, static_cast<int>(a.f), per_wave,             \
+                         b0 * kEdgeWaves);                                                                      \
+  } while (0)
     const dim3 grid(static_cast<unsigned>(nb));
-    const int64_t base = b0 * kWavesPerBlock;
-#define AS_ROWS(K) \
-  hipLaunchKernelGGL(K, grid, dim3(kBlock), 0, stream, a.crow, a.col, a.q, a.k, a.out, a.n, a.f, hub_threshold, base)
-    if (!vec) {
-      AS_ROWS((sddmm_rows_kernel<32, 1, false>));
-    } else {
-      switch (mf) {
-        case 1: AS_ROWS((sddmm_rows_kernel<8, 1, true>)); break;
-        case 2: AS_ROWS((sddmm_rows_kernel<8, 2, true>)); break;
-        case 3: AS_ROWS((sddmm_rows_kernel<8, 3, true>)); break;
-        case 4: AS_ROWS((sddmm_rows_kernel<8, 4, true>)); break;
-        case 5: AS_ROWS((sddmm_rows_kernel<8, 5, true>)); break;
-        case 6: AS_ROWS((sddmm_rows_kernel<8, 6, true>)); break;
-        case 7: AS_ROWS((sddmm_rows_kernel<8, 7, true>)); break;
-        default: AS_ROWS((sddmm_rows_kernel<8, 8, true>)); break;
+    const int nbl = static_cast<int>((a.f + 31) / 32);
+    const bool vec = a.f % 4 == 0;
+    if (a.f < 4) AS_E32(0, 1, 3);
+    else if (a.f == 32) AS_E32(0, 1, 0);
+    else if (a.f % 32 == 0) AS_E32(1, 1, 0);
+    else if (a.f < 32 && vec) AS_E32(0, 1, 1);
+    else if (a.f < 32) AS_E32(0, 1, 2);
+    else if (a.f < 64 && vec) AS_E32(0, 2, 1);
+    else if (a.f < 64) AS_E32(0, 2, 2);
+    else {
+      switch (nbl % 4) {
+        case 0: if (vec) AS_E32(4, 4, 1); else AS_E32(4, 4, 2); break;
+        case 1: if (vec) AS_E32(4, 1, 1); else AS_E32(4, 1, 2); break;
+        case 2: if (vec) AS_E32(4, 2, 1); else AS_E32(4, 2, 2); break;
+        default: if (vec) AS_E32(4, 3, 1); else AS_E32(4, 3, 2); break;
       }
     }
-#undef AS_ROWS
+#undef AS_E32
   }
-  return AS_OK;
 }
 
 // Workgroups given to the hub chunks of the scheduled kernel: one per chunk
@@ -285,36 +410,6 @@ int launch_sddmm_rows(const SddmmArgs& a, int64_t hub_threshold, hipStream_t str
 // threshold 256), and a pool much smaller than the chunk count leaves the
 // hub pass as a tail behind the light rows.
 constexpr int64_t kHubBlocksMax = 65536;
-
-int launch_sddmm_scheduled(const SddmmArgs& a, int waves, int64_t hub_threshold, int64_t item_upper,
-                           const int32_t* order, const int32_t* counts, const int32_t* chunk_off, hipStream_t stream) {
-  const int64_t hub_blocks = item_upper < kHubBlocksMax ? item_upper : kHubBlocksMax;
-  const int64_t blocks = hub_blocks + (a.n + waves - 1) / waves;
-  const dim3 block(static_cast<unsigned>(waves * kWave));
-  for (int64_t b0 = 0; b0 < blocks; b0 += kMaxBlocksPerLaunch) {
-    const int64_t nb = blocks - b0 < kMaxBlocksPerLaunch ? blocks - b0 : kMaxBlocksPerLaunch;
-    const dim3 grid(static_cast<unsigned>(nb));
-#define AS_SCHED(K)                                                                                             \
-  hipLaunchKernelGGL(K, grid, block, 0, stream, a.crow, a.col, a.q, a.k, a.out, a.n, a.f, hub_threshold, order, \
-                     counts, chunk_off, hub_blocks, b0)
-    if (!vec_ok(a)) {
-      AS_SCHED((sddmm_scheduled_kernel<32, 1, false>));
-    } else {
-      switch (static_cast<int>(a.f / 32)) {
-        case 1: AS_SCHED((sddmm_scheduled_kernel<8, 1, true>)); break;
-        case 2: AS_SCHED((sddmm_scheduled_kernel<8, 2, true>)); break;
-        case 3: AS_SCHED((sddmm_scheduled_kernel<8, 3, true>)); break;
-        case 4: AS_SCHED((sddmm_scheduled_kernel<8, 4, true>)); break;
-        case 5: AS_SCHED((sddmm_scheduled_kernel<8, 5, true>)); break;
-        case 6: AS_SCHED((sddmm_scheduled_kernel<8, 6, true>)); break;
-        case 7: AS_SCHED((sddmm_scheduled_kernel<8, 7, true>)); break;
-        default: AS_SCHED((sddmm_scheduled_kernel<8, 8, true>)); break;
-      }
-    }
-#undef AS_SCHED
-  }
-  return AS_OK;
-}
 
 // ---- bf16 / fp16 SDDMM -------------------------------------------------------
 // out[e] = the fp64 sum of the exact products q[row(e), f]·k[col(e), f],
@@ -622,8 +717,6 @@ void launch_sddmm16(const Sddmm16Args& a, int waves, int64_t hub_threshold, int6
 #endif
 constexpr int64_t kEdgeBlocksPerWave = AS_SDDMM16_EDGE_BLOCKS;
 constexpr int64_t kEdgesPerWave = kWave * kEdgeBlocksPerWave;
-constexpr int kEdgeWaves = 4;  // waves per workgroup
-
 int64_t edge_waves(int64_t nnz) { return (nnz + kEdgesPerWave - 1) / kEdgesPerWave; }
 
 size_t sddmm_edges_ws(int64_t nnz) {
@@ -645,37 +738,6 @@ __global__ __launch_bounds__(256) void edge_wave_rows_kernel(const int64_t* __re
     else hi = mid - 1;
   }
   rows[w] = static_cast<int32_t>(lo);
-}
-
-// Lane i: the row of edge b + min(i, cnt - 1), given r, the row of edge b.
-// Every lane of the wave must be active.  The rounds end at the last row
-// whatever crow holds, and the result is clamped to [0, n).
-__device__ __forceinline__ int block_edge_rows(const int64_t* __restrict__ crow, int64_t n, int64_t b, int cnt,
-                                               int64_t r) {
-  const int lane = lane_id();
-  const int i = lane < cnt ? lane : cnt - 1;
-  int row = -1;
-  for (int64_t rr = r;; rr += kWave) {
-    // rel: where row rr + lane ends (row n - 1 for lanes past it), relative
-    // to b, clamped to [0, 64]
-    const int64_t left = n - 1 - rr;  // >= 0
-    const int lim = left < kWave ? static_cast<int>(left) : kWave;
-    const int64_t d = crow[rr + 1 + (lane < lim ? lane : lim)] - b;
-    const int rel = d < 0 ? 0 : (d > kWave ? kWave : static_cast<int>(d));
-    // pos = #{l : rel_l <= i}, the ends being non-decreasing in l
-    int pos = 0;
-#pragma unroll
-    for (int s = kWave / 2; s >= 1; s >>= 1) {
-      const int v = __builtin_amdgcn_ds_bpermute((pos + s - 1) * 4, rel);
-      pos = v <= i ? pos + s : pos;
-    }
-    const int rel_last = __builtin_amdgcn_readlane(rel, kWave - 1);
-    if (pos == kWave - 1 && rel_last <= i) pos = kWave;
-    if (row < 0 && pos < kWave) row = static_cast<int>(rr + pos);
-    if (rel_last >= cnt || rr + kWave >= n) break;
-  }
-  const int last = static_cast<int>(n - 1);
-  return row < 0 || row > last ? last : row;
 }
 
 // Byte offset of 16-byte chunk lane_off of row `row` of a [*, F] matrix.
@@ -917,17 +979,22 @@ size_t sddmm_split_ws(int64_t n) {
 
 extern "C" {
 
-int as_sddmm_csr_f32(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,
-                     int64_t n, int64_t nnz, int64_t f, void* stream) {
+int as_sddmm_csr_edges_f32(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,
+                           int64_t n, int64_t n_keys, int64_t nnz, int64_t f, void* stream) {
   as::clear_error();
+  if (n_keys > INT32_MAX) return as::fail(AS_ERR_INVALID_ARGUMENT, "n_keys exceeds kernel index range");
   as::SddmmArgs a{crow, col, query, key, out, n, f};
   int st = as::validate_sddmm(a, nnz);
   if (st != AS_OK) return st;
   if (n == 0 || nnz == 0) return AS_OK;
   if (f == 0) return as::fail(AS_ERR_UNSUPPORTED, "SDDMM with zero features is handled by the caller");
-  st = as::launch_sddmm_rows(a, INT64_MAX, static_cast<hipStream_t>(stream));
-  if (st != AS_OK) return st;
+  as::launch_sddmm_edges(a, nnz, n_keys, static_cast<hipStream_t>(stream));
   return as::check_launch("sddmm_csr");
+}
+
+int as_sddmm_csr_f32(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,
+                     int64_t n, int64_t nnz, int64_t f, void* stream) {
+  return as_sddmm_csr_edges_f32(crow, col, query, key, out, n, -1, nnz, f, stream);
 }
 
 size_t as_sddmm_split_workspace_bytes(int64_t n) { return as::sddmm_split_ws(n < 0 ? 0 : n); }
@@ -948,28 +1015,8 @@ int as_sddmm_csr_split_f32(const int64_t* crow, const int64_t* col, const float*
   if (workspace == nullptr || workspace_bytes < as::sddmm_split_ws(n))
     return as::fail(AS_ERR_WORKSPACE, "split SDDMM needs %zu workspace bytes, got %zu", as::sddmm_split_ws(n),
                     workspace_bytes);
-  const hipStream_t s = static_cast<hipStream_t>(stream);
-  char* ws = static_cast<char*>(workspace);
-  int32_t* order = reinterpret_cast<int32_t*>(ws);
-  const size_t order_bytes = as::align_up(static_cast<size_t>(n) * sizeof(int32_t), 256);
-  int32_t* counts = reinterpret_cast<int32_t*>(ws + order_bytes);
-  void* bin_ws = ws + order_bytes + 256;
-  int32_t* chunk_off = reinterpret_cast<int32_t*>(ws + as::spmm_split_workspace_bytes(n));
-
-  int64_t heavy_upper = nnz / hub_threshold;
-  if (heavy_upper > n) heavy_upper = n;
-  if (heavy_upper == 0) {
-    // no row can reach the threshold: the row kernel covers everything
-    st = as::launch_sddmm_rows(a, hub_threshold, s);
-    if (st != AS_OK) return st;
-    return as::check_launch("sddmm_csr_split");
-  }
-  st = as::launch_bin_rows(crow, n, hub_threshold, 1, 1, order, counts, bin_ws, s);
-  if (st != AS_OK) return st;
-  hipLaunchKernelGGL(as::hub_chunk_scan_kernel, dim3(1), dim3(1024), 0, s, crow, order, counts, chunk_off);
-  const int64_t item_upper = nnz / as::kChunkEdges + heavy_upper;
-  st = as::launch_sddmm_scheduled(a, waves_per_block, hub_threshold, item_upper, order, counts, chunk_off, s);
-  if (st != AS_OK) return st;
+  // every schedule gives the same bits, and the blocks of edges need none
+  as::launch_sddmm_edges(a, nnz, -1, static_cast<hipStream_t>(stream));
   return as::check_launch("sddmm_csr_split");
 }
 

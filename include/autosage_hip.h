@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define AS_ABI_VERSION 9
+#define AS_ABI_VERSION 10
 
 typedef enum as_status {
   AS_OK = 0,
@@ -439,19 +439,28 @@ int as_csr_row_softmax_backward(const int64_t* crow, const void* probs, const vo
  * Replaces sddmm_csr (csrc/sddmm_csr_op.cu:108-134), op schema :192.
  * The dot product uses the reference kernel's summation order
  * (32 lane-strided fma chains, then a 16/8/4/2/1 tree,
- * csrc/sddmm_csr_op.cu:12-17,39-49). */
+ * csrc/sddmm_csr_op.cu:12-17,39-49).  One launch over blocks of 64 edges in
+ * CSR order, whatever the rows; no workspace. */
 int as_sddmm_csr_f32(const int64_t* crow, const int64_t* col,
                      const float* query, const float* key, float* out,
                      int64_t n, int64_t nnz, int64_t f, void* stream);
+
+/* as_sddmm_csr_f32 for a key of n_keys rows (n for a square graph; more for a
+ * row shard against the whole key), which must cover every column: knowing
+ * them lets the kernel use 32-bit offsets where they fit.  n_keys < 0: not
+ * known.  The same bits. */
+int as_sddmm_csr_edges_f32(const int64_t* crow, const int64_t* col,
+                           const float* query, const float* key, float* out,
+                           int64_t n, int64_t n_keys, int64_t nnz, int64_t f,
+                           void* stream);
 
 /* Bytes of workspace as_sddmm_csr_split_f32 needs for n rows. */
 size_t as_sddmm_split_workspace_bytes(int64_t n);
 
 /* Degree-split SDDMM.  Replaces sddmm_csr_split
- * (csrc/sddmm_csr_op.cu:136-187), op schema :193-195: rows with degree
- * < hub_threshold go to the row kernel, the rest are cut into edge chunks
- * spread over workgroups of waves_per_block waves.  Bit-identical to
- * as_sddmm_csr_f32. */
+ * (csrc/sddmm_csr_op.cu:136-187), op schema :193-195.  The settings and the
+ * workspace are checked; the product runs as as_sddmm_csr_f32, whose blocks of
+ * edges spread rows of any length without a split, with the same bits. */
 int as_sddmm_csr_split_f32(const int64_t* crow, const int64_t* col,
                            const float* query, const float* key, float* out,
                            int64_t n, int64_t nnz, int64_t f,
