@@ -262,6 +262,13 @@ def _fslice_eligible(crow, col, x, config: SchedulerConfig) -> bool:
     return config.full_graph_check and fslice_suits(crow, col, x, config.feature_slices)
 
 
+def fslice_large(crow, col, x) -> bool:
+    """X beyond the L2s and rows long on average: where XCD-local gathers pay
+    on any graph (no look at the rows themselves)."""
+    n = crow.numel() - 1
+    return x.numel() * x.element_size() >= _COLSLICE_MIN_X_BYTES and col.numel() >= _COLSLICE_MIN_MEAN_DEGREE * n
+
+
 def fslice_suits(crow, col, x, mode: str) -> bool:
     """Whether the feature-sliced SpMM is worth running for this graph and X:
     graphs whose X is beyond the L2s with long rows on average, or with a
@@ -274,8 +281,7 @@ def fslice_suits(crow, col, x, mode: str) -> bool:
     if mode == "auto":
         from ._native import row_counts
 
-        large = x.numel() * x.element_size() >= _COLSLICE_MIN_X_BYTES and col.numel() >= _COLSLICE_MIN_MEAN_DEGREE * n
-        if not large and row_counts(crow, _COLSLICE_HUB_DEGREE, 0)[0] == 0:
+        if not fslice_large(crow, col, x) and row_counts(crow, _COLSLICE_HUB_DEGREE, 0)[0] == 0:
             return False
     return True
 

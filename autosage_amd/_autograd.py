@@ -57,14 +57,10 @@ def _build_transpose(crow: torch.Tensor, col: torch.Tensor) -> tuple[torch.Tenso
     return crow_t, rows.index_select(0, perm).contiguous(), perm
 
 
-# The backward SpMMs run on the degree-split schedule when the graph has hub
-# rows: bit-identical to the whole-graph kernel (CSR order per output), but
-# hub rows are split across waves, which matters on skewed graphs (one wave
-# per 200k-edge row is several times slower).  Without hub rows the
-# whole-graph SpMM runs (memoised per-graph row count, one launch).
-_HUB_THRESHOLD = 1024
-
-
+# The backward SpMMs run on the feature-sliced kernel where X is beyond the L2s
+# and rows are long (or where it is forced on), else on the whole-graph kernel,
+# which gives long rows workgroups of their own: the same bits (CSR order per
+# output) and no host sync on a new graph's transpose.
 def _spmm(crow, col, val, x, sliced: bool = False):
     if x.dtype != torch.float32:
         # bf16 / fp16: the rounded SpMM, the same bits on any schedule
@@ -75,25 +71,21 @@ def _spmm(crow, col, val, x, sliced: bool = False):
         # columns in ascending order, so it needs no row-sorted copy
         return torch.ops.autosage.spmm_csr_colslice(crow, col, val, x)
     if _feature_slices_pay(crow, col, x):
-        # the same bits as the schedules below, XCD-local on large graphs
+        # the same bits, XCD-local on large graphs
         return torch.ops.autosage.spmm_csr_fslice(crow, col, val, x)
-    from ._native import row_counts
-
-    if row_counts(crow, _HUB_THRESHOLD, 0)[0] == 0:
-        # no hub row: the whole-graph kernel, one launch without binning
-        return torch.ops.autosage.spmm_csr(crow, col, val, x)
-    tile = 64 if x.size(1) <= 64 else 128
-    return torch.ops.autosage.spmm_csr_split(crow, col, val, x, tile, 2, _HUB_THRESHOLD)
+    return torch.ops.autosage.spmm_csr(crow, col, val, x)
 
 
 def _feature_slices_pay(crow, col, x) -> bool:
-    """The feature-sliced SpMM for a backward product when the forward
-    scheduler would time it (``auto``: X beyond the L2s with long rows, or a
-    hub row) or it is forced on."""
-    from ._auto import fslice_suits
+    """The feature-sliced SpMM for a backward product: X beyond the L2s with
+    long rows on average (``auto``), every graph with edges (``on``)."""
+    from ._auto import fslice_large, fslice_suits
     from .config import SchedulerConfig
 
-    return fslice_suits(crow, col, x, SchedulerConfig.from_env().feature_slices)
+    mode = SchedulerConfig.from_env().feature_slices
+    if mode == "auto":
+        return fslice_large(crow, col, x) and fslice_suits(crow, col, x, mode)
+    return fslice_suits(crow, col, x, mode)
 
 
 def _column_slices_allowed() -> bool:

@@ -89,6 +89,15 @@ class GraphMemo:
         self.put(tensors, extra, value, key=key)
         return value
 
+    def peek(self, tensors: Sequence[torch.Tensor], extra: Hashable) -> Any:
+        """The memoised value, or None; computes nothing and records no
+        stream (for values that hold no device tensors)."""
+        with self._lock:
+            hit = self._entries.get(self._key(tensors, extra))
+            if hit is not None and all(ref() is t for ref, t in zip(hit[0], tensors)):
+                return hit[1]
+        return None
+
     @staticmethod
     def _current_stream(device: torch.device):
         return torch.cuda.current_stream(device)

@@ -44,6 +44,11 @@ _SIGNATURES = {
     "as_last_error": (ctypes.c_char_p, []),
     "as_abi_version": (_c_int, []),
     "as_spmm_csr_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr]),
+    "as_spmm_csr_rows_f32": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_ptr],
+    ),
+    "as_spmm_long_row": (_c_i64, []),
     "as_bin_workspace_bytes": (_c_size, [_c_i64]),
     "as_bin_rows_by_degree": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "as_spmm_split_workspace_bytes": (_c_size, [_c_i64]),
@@ -354,11 +359,36 @@ def spmm_csr_impl(crow, col, val, x):
     if n == 0 or f == 0:
         return y
     with _on(x.device):
-        status = library().as_spmm_csr_f32(
-            _ptr(crow), _ptr(col), _ptr(val), _ptr(x), _ptr(y), n, col.numel(), f, int(_env_vec4()), _stream(x.device)
+        status = library().as_spmm_csr_rows_f32(
+            _ptr(crow), _ptr(col), _ptr(val), _ptr(x), _ptr(y), n, n, col.numel(), f, int(_env_vec4()),
+            int(_even_rows(crow, col, f)), _stream(x.device),
         )
     _raise(status, "autosage::spmm_csr")
     return y
+
+
+# fp32 spmm_csr asks for the longest row (once per graph: one host sync,
+# memoised) where it changes the launch by more than the question costs: wide
+# rows of 12 edges or more on graphs of this many edges.
+_EVEN_ROWS_MIN_NNZ = 1 << 19
+
+
+def _even_rows(crow: torch.Tensor, col: torch.Tensor, f: int) -> bool:
+    """Whether the graph is known to have no row of as_spmm_long_row() edges
+    (the same bits either way).  A stream capture takes no sync: only what
+    an earlier call found out counts there."""
+    n = crow.numel() - 1
+    if not 32 < f <= 256 or col.numel() < max(_EVEN_ROWS_MIN_NNZ, 12 * n):
+        return False
+
+    def compute() -> int:
+        return int((crow[1:] - crow[:-1]).amax().item())
+
+    if torch.cuda.is_current_stream_capturing():
+        longest = _ROW_COUNT_MEMO.peek((crow,), "longest")
+    else:
+        longest = _ROW_COUNT_MEMO.get((crow,), "longest", compute)
+    return longest is not None and longest < library().as_spmm_long_row()
 
 
 def spmm_csr_split_impl(crow, col, val, x, feature_tile, warps_per_block, hub_threshold):
@@ -622,7 +652,7 @@ def spmm_csr_rect_impl(crow, col, val, x, exact: bool = False):
     larger graph (its rows, crow rebased to 0, the columns unchanged) with
     the whole X.
 
-    ``exact``: fp32 only, one wave per row in CSR order (the sequential
+    ``exact``: fp32 only, the rows in CSR order (the sequential
     fp32 product of ``spmm_csr``, bit-identical to the same rows of the whole
     graph's product).  Otherwise the column-sliced schedule: fp32 with fp64
     partials per column slice, 16-bit rounded once; the slices cut the
@@ -639,9 +669,9 @@ def spmm_csr_rect_impl(crow, col, val, x, exact: bool = False):
         validate_csr(crow, col, n_cols)
     if exact:
         with _on(x.device):
-            status = library().as_spmm_csr_f32(
-                _ptr(crow), _ptr(col), _ptr(val), _ptr(x), _ptr(y), n, col.numel(), f, int(_env_vec4()),
-                _stream(x.device),
+            status = library().as_spmm_csr_rows_f32(
+                _ptr(crow), _ptr(col), _ptr(val), _ptr(x), _ptr(y), n, n_cols, col.numel(), f, int(_env_vec4()),
+                int(_even_rows(crow, col, f)), _stream(x.device),
             )
         _raise(status, "autosage row-shard SpMM")
         return y

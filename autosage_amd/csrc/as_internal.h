@@ -46,6 +46,12 @@ inline int validate_spmm(const int64_t* crow, const int64_t* col, const void* x,
   return AS_OK;
 }
 
+// fp32 SpMM in CSR order: lane groups on short rows, workgroups on rows of at
+// least kSpmmLongRow edges (spmm_groups.hip).  f >= 4, n and nnz > 0; n_cols < 0: not known.
+constexpr int64_t kSpmmLongRow = 256;
+void launch_spmm_groups(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y, int64_t n,
+                        int64_t n_cols, int64_t nnz, int64_t f, hipStream_t stream);
+
 // Degree binning (binning.hip).
 constexpr int kBinRowsPerThread = 4;
 constexpr int kBinTile = kBlock * kBinRowsPerThread;

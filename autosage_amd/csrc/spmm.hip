@@ -481,18 +481,34 @@ size_t spmm_split_workspace_bytes(int64_t n) {
 
 extern "C" {
 
-int as_spmm_csr_f32(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y, int64_t n,
-                    int64_t nnz, int64_t f, int vec4, void* stream) {
+int as_spmm_csr_rows_f32(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y, int64_t n,
+                         int64_t n_cols, int64_t nnz, int64_t f, int vec4, int even_rows, void* stream) {
   as::clear_error();
   int st = as::validate_spmm(crow, col, x, y, n, nnz, f);
   if (st != AS_OK) return st;
   if (n == 0 || f == 0) return AS_OK;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  // one wave per row is 1-10 % faster than lane groups on even rows of 33 to 256
+  // features and 12 edges or more (1M rows, 16.8M edges: F = 47 731 against 798 us, F = 64
+  // 642 / 658, F = 128 1217 / 1298; narrower F = 32 494 / 360, wider F = 300 4069 / 3845,
+  // 4 edges a row F = 47 71 / 45), but up to 3 times slower on graphs with long rows
+  const bool wide = nnz >= as::kSubwaveMaxMeanDegree * n && f > 32 && f <= 256 && (f <= 64 || f % 2 == 0);
+  if (vec4 != 0 && f >= 4 && nnz > 0 && !(even_rows != 0 && wide)) {
+    as::launch_spmm_groups(crow, col, val, x, y, n, n_cols, nnz, f, s);
+    return as::check_launch("spmm_csr");
+  }
   const as::SpmmArgs a{crow, col, val, x, y, n, f};
   const int layout = as::pick_layout(a, nnz, 128, vec4 != 0);
   if (val != nullptr) as::launch_rows<true>(a, layout, s);
   else as::launch_rows<false>(a, layout, s);
   return as::check_launch("spmm_csr");
+}
+
+int64_t as_spmm_long_row(void) { return as::kSpmmLongRow; }
+
+int as_spmm_csr_f32(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y, int64_t n,
+                    int64_t nnz, int64_t f, int vec4, void* stream) {
+  return as_spmm_csr_rows_f32(crow, col, val, x, y, n, -1, nnz, f, vec4, 0, stream);
 }
 
 size_t as_spmm_split_workspace_bytes(int64_t n) { return as::spmm_split_workspace_bytes(n < 0 ? 0 : n); }

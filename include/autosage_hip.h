@@ -75,6 +75,20 @@ int as_spmm_csr_f32(const int64_t* crow, const int64_t* col, const float* val,
                     const float* x, float* y, int64_t n, int64_t nnz,
                     int64_t f, int vec4, void* stream);
 
+/* as_spmm_csr_f32 (the same bits) with what the caller knows of the graph:
+ * n_cols, the rows of X, which must cover every column (32-bit offsets where
+ * they fit; < 0: not known), and even_rows != 0 where no row has
+ * as_spmm_long_row() edges or more.  Short rows run in lane groups and long
+ * ones on workgroups of their own; wide rows of a graph known to be even take
+ * one wave each, a few percent faster there. */
+int as_spmm_csr_rows_f32(const int64_t* crow, const int64_t* col, const float* val,
+                         const float* x, float* y, int64_t n, int64_t n_cols,
+                         int64_t nnz, int64_t f, int vec4, int even_rows,
+                         void* stream);
+
+/* Degree from which as_spmm_csr_rows_f32 gives a row to a workgroup. */
+int64_t as_spmm_long_row(void);
+
 /* Bytes of workspace as_bin_rows_by_degree needs for n rows. */
 size_t as_bin_workspace_bytes(int64_t n);
 
