@@ -23,8 +23,8 @@ backward formulas built from the same native kernels:
   float32, bf16 or fp16, fp32 sums), with no nnz-sized intermediate.
 
 The transposed CSR (rows of Aᵀ list the source rows in ascending order, a
-stable sort of the edges by column) is built with torch ops and memoised per
-live (crow, col) tensor pair, like the schedule keys.  Every product is
+stable sort of the edges by column) is built once and memoised per live
+(crow, col) tensor pair, like the schedule keys.  Every product is
 deterministic: the same inputs give the same bits.
 """
 
@@ -49,6 +49,11 @@ def csr_transpose(crow: torch.Tensor, col: torch.Tensor) -> tuple[torch.Tensor, 
 
 def _build_transpose(crow: torch.Tensor, col: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     n = crow.numel() - 1
+    if crow.is_cuda:
+        from . import _native
+
+        if _native.csr_build_supported(crow, col, n):
+            return _native.csr_transpose(crow, col)
     counts = (crow[1:] - crow[:-1]).to(torch.long)
     rows = torch.repeat_interleave(torch.arange(n, device=crow.device, dtype=torch.long), counts)
     perm = col.argsort(stable=True)

@@ -49,6 +49,11 @@ _SIGNATURES = {
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_ptr],
     ),
     "as_spmm_long_row": (_c_i64, []),
+    "as_csr_build_workspace_bytes": (_c_size, [_c_i64, _c_i64]),
+    "as_csr_from_edges": (
+        _c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
+    "as_csr_transpose": (
+        _c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "as_bin_workspace_bytes": (_c_size, [_c_i64]),
     "as_bin_rows_by_degree": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "as_spmm_split_workspace_bytes": (_c_size, [_c_i64]),
@@ -1323,6 +1328,50 @@ def induced_sample(crow: torch.Tensor, col: torch.Tensor, val: Optional[torch.Te
                                           _ptr(new_col), _ptr(new_val), _ptr(ws), ws.numel(), stream),
                "induced_sample")
     return new_crow, new_col, new_val
+
+
+_is_wrapped = getattr(torch._C._functorch, "is_functorch_wrapped_tensor", None)
+
+
+def csr_build_supported(rows: torch.Tensor, cols: torch.Tensor, n: int) -> bool:
+    """Whether ``csr_from_edges`` / ``csr_transpose`` take these ids: plain
+    contiguous int64 CUDA vectors of the sizes the native sort covers, outside
+    tracing, functorch transforms and stream capture (the sort may record
+    memsets), which keep the torch composition."""
+    return (type(rows) is torch.Tensor and type(cols) is torch.Tensor and rows.is_cuda and cols.is_cuda
+            and rows.get_device() == cols.get_device()
+            and rows.dtype is torch.long and cols.dtype is torch.long and rows.dim() == 1 and cols.dim() == 1
+            and rows.is_contiguous() and cols.is_contiguous()
+            and 0 < n and 0 < cols.numel() and n + cols.numel() < 2**31 - 4097
+            and _LIB is not None and _is_wrapped is not None and not _is_wrapped(rows) and not _is_wrapped(cols)
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch.cuda.is_current_stream_capturing())
+
+
+def _csr_build(entry, first, second, n: int, edges: int, want_perm: bool):
+    device = first.device
+    lib = library()
+    ws = _workspace(lib.as_csr_build_workspace_bytes(n, edges), device)
+    crow = torch.empty(n + 1, dtype=torch.long, device=device)
+    col = torch.empty(edges, dtype=torch.long, device=device)
+    perm = torch.empty(edges, dtype=torch.long, device=device) if want_perm else None
+    with _on(device):
+        status = entry(_ptr(first), _ptr(second), n, edges, _ptr(crow), _ptr(col), _ptr(perm), _ptr(ws), ws.numel(),
+                       _stream(device))
+    _raise(status, "autosage CSR build")
+    return crow, col, perm
+
+
+def csr_from_edges(rows: torch.Tensor, cols: torch.Tensor, n: int, want_perm: bool = True):
+    """(crow, col, perm or None): the CSR of an edge list on the device, the
+    edges in a stable sort by row (see ``csr_build_supported``)."""
+    return _csr_build(library().as_csr_from_edges, rows, cols, int(n), rows.numel(), want_perm)
+
+
+def csr_transpose(crow: torch.Tensor, col: torch.Tensor):
+    """(crow_t, col_t, perm) of the transposed n x n CSR on the device, per
+    column the source rows in ascending order (see ``csr_build_supported``)."""
+    return _csr_build(library().as_csr_transpose, crow, col, crow.numel() - 1, col.numel(), True)
 
 
 def bin_rows_by_degree(crow: torch.Tensor, threshold: int) -> tuple[torch.Tensor, torch.Tensor]:

@@ -59,53 +59,6 @@ __global__ __launch_bounds__(1024) void hub_chunk_scan_kernel(const int64_t* __r
   if (threadIdx.x == 0) counts[2] = total;
 }
 
-// Lane i: the row of edge b + min(i, cnt - 1), given r, the row of edge b.
-// Every lane of the wave must be active.  The rounds end at the last row
-// whatever crow holds, and the result is clamped to [0, n).
-__device__ __forceinline__ int block_edge_rows(const int64_t* __restrict__ crow, int64_t n, int64_t b, int cnt,
-                                               int64_t r) {
-  const int lane = lane_id();
-  const int i = lane < cnt ? lane : cnt - 1;
-  int row = -1;
-  for (int64_t rr = r;; rr += kWave) {
-    // rel: where row rr + lane ends (row n - 1 for lanes past it), relative
-    // to b, clamped to [0, 64]
-    const int64_t left = n - 1 - rr;  // >= 0
-    const int lim = left < kWave ? static_cast<int>(left) : kWave;
-    const int64_t d = crow[rr + 1 + (lane < lim ? lane : lim)] - b;
-    const int rel = d < 0 ? 0 : (d > kWave ? kWave : static_cast<int>(d));
-    // pos = #{l : rel_l <= i}, the ends being non-decreasing in l
-    int pos = 0;
-#pragma unroll
-    for (int s = kWave / 2; s >= 1; s >>= 1) {
-      const int v = __builtin_amdgcn_ds_bpermute((pos + s - 1) * 4, rel);
-      pos = v <= i ? pos + s : pos;
-    }
-    const int rel_last = __builtin_amdgcn_readlane(rel, kWave - 1);
-    if (pos == kWave - 1 && rel_last <= i) pos = kWave;
-    if (row < 0 && pos < kWave) row = static_cast<int>(rr + pos);
-    if (rel_last >= cnt || rr + kWave >= n) break;
-  }
-  const int last = static_cast<int>(n - 1);
-  return row < 0 || row > last ? last : row;
-}
-
-// The row holding edge e: the last r < n with crow[r] <= e (0 if none), by
-// the whole wave, 64 probes a step; ends after log64(n) steps whatever crow
-// holds.
-__device__ __forceinline__ int64_t wave_row_of_edge(const int64_t* __restrict__ crow, int64_t n, int64_t e) {
-  int64_t lo = 0;
-  int64_t hi = n;
-  while (hi - lo > 1) {
-    const int64_t step = (hi - lo + kWave - 1) / kWave;
-    const int64_t probe = lo + lane_id() * step;
-    const uint64_t below = __ballot(probe < hi && crow[probe] <= e);
-    if (below != 0) lo += static_cast<int64_t>(63 - __builtin_clzll(below)) * step;
-    hi = lo + step < hi ? lo + step : hi;
-  }
-  return lo;
-}
-
 // ---- fp32 SDDMM by blocks of edges ------------------------------------------
 // The edges in CSR order, 64 a block, whatever the rows; every output keeps
 // the reference's order (file comment).  8 lanes per edge and 8 edges per

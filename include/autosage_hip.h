@@ -89,6 +89,28 @@ int as_spmm_csr_rows_f32(const int64_t* crow, const int64_t* col, const float* v
 /* Degree from which as_spmm_csr_rows_f32 gives a row to a workgroup. */
 int64_t as_spmm_long_row(void);
 
+/* Bytes of workspace as_csr_from_edges and as_csr_transpose need; 0 where
+ * the sizes are out of range (n, edges >= 1, n + edges < 2^31 - 4096). */
+size_t as_csr_build_workspace_bytes(int64_t n, int64_t edges);
+
+/* The CSR of an edge list: the edges in a stable sort by `rows` (int64 ids in
+ * [0, n)), col[k] = cols[perm[k]], crow[r] = edges of rows below r.  The
+ * outputs of edge_index_to_csr (autosage/utils/csr.py:6-26), bit for bit;
+ * crow int64[n + 1], col int64[edges], perm int64[edges] or null.  An edge
+ * whose row id lies outside [0, n) is left behind the last row (crow[n]).
+ * No host sync; not for stream capture (the sort may record memsets). */
+int as_csr_from_edges(const int64_t* rows, const int64_t* cols, int64_t n,
+                      int64_t edges, int64_t* crow, int64_t* col, int64_t* perm,
+                      void* workspace, size_t workspace_bytes, void* stream);
+
+/* The transpose of an n x n CSR (no reference counterpart): per column the
+ * source rows in ascending order, col_t[k] = row of edge perm[k].  As
+ * as_csr_from_edges otherwise. */
+int as_csr_transpose(const int64_t* crow, const int64_t* col, int64_t n,
+                     int64_t nnz, int64_t* crow_t, int64_t* col_t,
+                     int64_t* perm, void* workspace, size_t workspace_bytes,
+                     void* stream);
+
 /* Bytes of workspace as_bin_rows_by_degree needs for n rows. */
 size_t as_bin_workspace_bytes(int64_t n);
 
