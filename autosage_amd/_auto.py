@@ -15,7 +15,7 @@ gfx950 changes:
   cached, so a replayed schedule is never slower than the baseline on the
   graph it was made for;
 * the CSR row softmax and the attention pipeline run as native kernels on the
-  GPU (``csr_attention_forward`` can fuse all three stages into one launch).
+  GPU (``csr_attention_forward`` can run all three stages in one call).
 """
 
 from __future__ import annotations
@@ -1014,8 +1014,8 @@ def _attention_colslice_eligible(crow, col, query, value, config: SchedulerConfi
 
 
 def _attention_variant(crow, col, q, k, v, scale: float) -> tuple[str, dict[str, Any]]:
-    """"fused" (the exact fused kernel) or "colslice" for this graph: the
-    column-sliced attention is timed against the fused kernel once per graph
+    """"fused" (the exact stages in one call) or "colslice" for this graph: the
+    column-sliced attention is timed against the exact one once per graph
     on the full graph when eligible, and the faster one is cached."""
     config = SchedulerConfig.from_env()
     if not _attention_colslice_eligible(crow, col, q, v, config):
@@ -1066,8 +1066,8 @@ def csr_attention_forward(
     the reference has no scale, i.e. scale = 1).
 
     On the GPU with ``fused`` (default: the ``AUTOSAGE_FUSED_ATTENTION``
-    switch, on) the three stages run as one native kernel: for float32 the
-    exact fused kernel or the column-sliced one, whichever a full-graph
+    switch, on) the three stages run as one native call: for float32 the
+    exact stages or the column-sliced kernel, whichever a full-graph
     timing picks; for bf16 / fp16 the column-sliced kernel in fp32 arithmetic
     with each output rounded once (when its widths fit: multiples of 8 up to
     512).  Otherwise the stages run as the scheduled SDDMM, the row softmax
@@ -1092,8 +1092,12 @@ def csr_attention_forward(
             raise RuntimeError("AutoSAGE native csr_attention is unavailable")
         v = value.contiguous()
         variant, decision = _attention_variant(crow_n, col_n, q, k, v, float(scale))
-        out = native_op("csr_attention" if variant == "fused" else "csr_attention_colslice")(
-            crow_n, col_n, q, k, v, float(scale))
+        if variant == "fused" and torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v)):
+            # the backward takes the probabilities (4 bytes an edge) from here
+            out = native_op("csr_attention_probs")(crow_n, col_n, q, k, v, float(scale))[0]
+        else:
+            out = native_op("csr_attention" if variant == "fused" else "csr_attention_colslice")(
+                crow_n, col_n, q, k, v, float(scale))
         info = {"operation": "attention", "schema_version": AUTOTUNE_SCHEMA_VERSION, "choice": "fused",
                 "from_cache": decision.get("from_cache", False)}
         return out, {"sddmm": {**info, "operation": "sddmm"}, "spmm": {**info, "operation": "spmm"}, "fused": True,

@@ -897,7 +897,8 @@ def csr_row_softmax_backward_impl(crow, probs, grad):
     return out
 
 
-def csr_attention_impl(crow, col, query, key, value, scale=1.0):
+def csr_attention_probs_impl(crow, col, query, key, value, scale=1.0):
+    """(out, probabilities per edge) of ``csr_attention``."""
     check_sddmm_inputs(crow, col, query, key)
     _maybe_validate(crow, col)
     _check(value.is_cuda and value.device == query.device, "value must be on the same CUDA device as query")
@@ -907,22 +908,24 @@ def csr_attention_impl(crow, col, query, key, value, scale=1.0):
     n, fqk = query.shape
     fv = value.size(1)
     nnz = col.numel()
-    out = torch.empty((n, fv), dtype=value.dtype, device=value.device)
-    if n == 0 or fv == 0:
-        return out
-    if fqk == 0 and nnz > 0:
+    if fqk == 0 and nnz > 0 and fv > 0:
         # all scores are zero: the softmax of each row is uniform
-        scores = torch.zeros(nnz, dtype=query.dtype, device=query.device)
-        return spmm_csr_impl(crow, col, csr_row_softmax_impl(crow, scores), value)
+        probs = csr_row_softmax_impl(crow, torch.zeros(nnz, dtype=query.dtype, device=query.device))
+        return spmm_csr_impl(crow, col, probs, value), probs
+    out = torch.empty((n, fv), dtype=value.dtype, device=value.device)
     lib = library()
-    ws = _workspace(lib.as_csr_attention_workspace_bytes(n, nnz), query.device)
+    ws = torch.empty(max(nnz, 1), dtype=torch.float32, device=query.device)  # scores, then probabilities
     with _on(query.device):
         status = lib.as_csr_attention_f32(
             _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(value), _ptr(out), n, nnz, fqk, fv, float(scale),
-            _ptr(ws), ws.numel(), _stream(query.device),
+            _ptr(ws), ws.numel() * 4, _stream(query.device),
         )
     _raise(status, "autosage::csr_attention")
-    return out
+    return out, ws[:nnz]
+
+
+def csr_attention_impl(crow, col, query, key, value, scale=1.0):
+    return csr_attention_probs_impl(crow, col, query, key, value, scale)[0]
 
 
 def attention_colslice_supported(query: torch.Tensor, value: torch.Tensor) -> bool:
@@ -1419,6 +1422,12 @@ _SCHEMAS = {
     "csr_attention": (
         "csr_attention(Tensor crow, Tensor col, Tensor query, Tensor key, Tensor value, float scale=1.0) -> Tensor",
         csr_attention_impl,
+    ),
+    # csr_attention with the probabilities, for a backward that does not sum the scores again
+    "csr_attention_probs": (
+        "csr_attention_probs(Tensor crow, Tensor col, Tensor query, Tensor key, Tensor value, float scale=1.0) "
+        "-> (Tensor, Tensor)",
+        csr_attention_probs_impl,
     ),
     "csr_attention_colslice": (
         "csr_attention_colslice(Tensor crow, Tensor col, Tensor query, Tensor key, Tensor value, float scale=1.0) "

@@ -52,6 +52,14 @@ constexpr int64_t kSpmmLongRow = 256;
 void launch_spmm_groups(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y, int64_t n,
                         int64_t n_cols, int64_t nnz, int64_t f, hipStream_t stream);
 
+// The stages of the exact attention: scale times the SDDMM of a square graph
+// (sddmm.hip; f, n and nnz > 0), and the SpMM with one wave per row for what
+// the lane groups do not take (spmm.hip; arguments checked by the caller).
+void launch_sddmm_scaled(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,
+                         int64_t n, int64_t nnz, int64_t f, float scale, hipStream_t stream);
+void launch_spmm_wave_rows(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y,
+                           int64_t n, int64_t nnz, int64_t f, bool vec4, hipStream_t stream);
+
 // Degree binning (binning.hip).
 constexpr int kBinRowsPerThread = 4;
 constexpr int kBinTile = kBlock * kBinRowsPerThread;

@@ -262,8 +262,8 @@ constexpr int kEdgeWaves = 4;  // waves per workgroup
 template <int CB, int LAST, int TAIL, bool OFF32>
 __global__ __launch_bounds__(kEdgeWaves * kWave) __attribute__((amdgpu_waves_per_eu(4))) void sddmm_edges_kernel(
     const int64_t* __restrict__ crow, const int64_t* __restrict__ col, const float* __restrict__ query,
-    const float* __restrict__ key, float* __restrict__ out, int64_t n, int64_t nnz, int F, int64_t per_wave,
-    int64_t wave_base) {
+    const float* __restrict__ key, float* __restrict__ out, int64_t n, int64_t nnz, int F, float scale,
+    int64_t per_wave, int64_t wave_base) {
   const int64_t w = wave_base + static_cast<int64_t>(blockIdx.x) * kEdgeWaves + wave_in_block();
   const int64_t b0 = uniform_i64(w * per_wave);
   if (b0 >= nnz) return;  // wave-uniform
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(kEdgeWaves * kWave) __attribute__((amdgpu_waves_per
       r = __builtin_amdgcn_readlane(my_row, cnt - 1);
       d = edge_block_dots<CB, LAST, TAIL, OFF32, false>(kb, qb, F, my_c, my_row);
     }
-    if (lane < cnt) out[b + lane] = d;
+    if (lane < cnt) out[b + lane] = d * scale;  // scale 1: the dot product's bits
   }
 }
 
@@ -312,7 +312,7 @@ constexpr int64_t kWideRow = 96;
 
 // n_keys: rows of the key, or -1 where the caller does not know them (64-bit
 // offsets then).
-void launch_sddmm_edges(const SddmmArgs& a, int64_t nnz, int64_t n_keys, hipStream_t s) {
+void launch_sddmm_edges(const SddmmArgs& a, int64_t nnz, int64_t n_keys, float scale, hipStream_t s) {
   int64_t per = nnz / (kFillWaves * kWave);
   const bool in_order = a.f >= kWideRow && nnz < kShortRowDegree * a.n;
   per = per < 1 || in_order ? 1 : (per > kMaxEdgeBlocks ? kMaxEdgeBlocks : per);
@@ -323,15 +323,16 @@ void launch_sddmm_edges(const SddmmArgs& a, int64_t nnz, int64_t n_keys, hipStre
   const bool off32 = n_keys > 0 && rows * a.f * 4 <= (int64_t(1) << 32);
   for (int64_t b0 = 0; b0 < blocks; b0 += kMaxBlocksPerLaunch) {
     const int64_t nb = blocks - b0 < kMaxBlocksPerLaunch ? blocks - b0 : kMaxBlocksPerLaunch;
-#define AS_E32(CB, LAST, TAIL)                                                                                    \
-  do {                                                                                                          \
-    if (off32)                                                                                                  \
+#define AS_E32(CB, LAST, TAIL)                                                                                     \
+  do {                                                                                                           \
+    if (off32)                                                                                                   \
       hipLaunchKernelGGL((sddmm_edges_kernel<CB, LAST, TAIL, true>), grid, dim3(kEdgeWaves * kWave), 0, s, a.crow, \
-                         a.col, a.q, a.k, a.out, a.n, nnz, static_cast<int>(a.f), per_wave, b0 * kEdgeWaves);   \
-    else                                                                                                        \
-      hipLaunchKernelGGL((sddmm_edges_kernel<CB, LAST, TAIL, false>), grid, dim3(kEdgeWaves * kWave), 0, s,     \
-                         a.crow, a.col, a.q, a.k, a.out, a.n, nnz, static_cast<int>(a.f), per_wave,             \
-                         b0 * kEdgeWaves);                                                                      \
+                         a.col, a.q, a.k, a.out, a.n, nnz, static_cast<int>(a.f), scale, per_wave,               \
+                         b0 * kEdgeWaves);                                                                       \
+    else                                                                                                         \
+      hipLaunchKernelGGL((sddmm_edges_kernel<CB, LAST, TAIL, false>), grid, dim3(kEdgeWaves * kWave), 0, s,      \
+                         a.crow, a.col, a.q, a.k, a.out, a.n, nnz, static_cast<int>(a.f), scale, per_wave,       \
+                         b0 * kEdgeWaves);                                                                       \
   } while (0)
     const dim3 grid(static_cast<unsigned>(nb));
     const int nbl = static_cast<int>((a.f + 31) / 32);
@@ -928,6 +929,11 @@ size_t sddmm_split_ws(int64_t n) {
 
 }  // namespace
 
+void launch_sddmm_scaled(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,
+                         int64_t n, int64_t nnz, int64_t f, float scale, hipStream_t s) {
+  launch_sddmm_edges(SddmmArgs{crow, col, query, key, out, n, f}, nnz, n, scale, s);
+}
+
 }  // namespace as
 
 extern "C" {
@@ -941,7 +947,7 @@ int as_sddmm_csr_edges_f32(const int64_t* crow, const int64_t* col, const float*
   if (st != AS_OK) return st;
   if (n == 0 || nnz == 0) return AS_OK;
   if (f == 0) return as::fail(AS_ERR_UNSUPPORTED, "SDDMM with zero features is handled by the caller");
-  as::launch_sddmm_edges(a, nnz, n_keys, static_cast<hipStream_t>(stream));
+  as::launch_sddmm_edges(a, nnz, n_keys, 1.f, static_cast<hipStream_t>(stream));
   return as::check_launch("sddmm_csr");
 }
 
@@ -969,7 +975,7 @@ int as_sddmm_csr_split_f32(const int64_t* crow, const int64_t* col, const float*
     return as::fail(AS_ERR_WORKSPACE, "split SDDMM needs %zu workspace bytes, got %zu", as::sddmm_split_ws(n),
                     workspace_bytes);
   // every schedule gives the same bits, and the blocks of edges need none
-  as::launch_sddmm_edges(a, nnz, -1, static_cast<hipStream_t>(stream));
+  as::launch_sddmm_edges(a, nnz, -1, 1.f, static_cast<hipStream_t>(stream));
   return as::check_launch("sddmm_csr_split");
 }
 

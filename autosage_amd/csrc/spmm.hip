@@ -470,6 +470,14 @@ void launch_sched_v(int hv, int layout, const SpmmArgs& a, const SchedLaunch& l,
 
 }  // namespace
 
+void launch_spmm_wave_rows(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y,
+                           int64_t n, int64_t nnz, int64_t f, bool vec4, hipStream_t s) {
+  const SpmmArgs a{crow, col, val, x, y, n, f};
+  const int layout = pick_layout(a, nnz, 128, vec4);
+  if (val != nullptr) launch_rows<true>(a, layout, s);
+  else launch_rows<false>(a, layout, s);
+}
+
 constexpr int kSplitBuckets = 8;
 
 size_t spmm_split_workspace_bytes(int64_t n) {
@@ -497,10 +505,7 @@ int as_spmm_csr_rows_f32(const int64_t* crow, const int64_t* col, const float* v
     as::launch_spmm_groups(crow, col, val, x, y, n, n_cols, nnz, f, s);
     return as::check_launch("spmm_csr");
   }
-  const as::SpmmArgs a{crow, col, val, x, y, n, f};
-  const int layout = as::pick_layout(a, nnz, 128, vec4 != 0);
-  if (val != nullptr) as::launch_rows<true>(a, layout, s);
-  else as::launch_rows<false>(a, layout, s);
+  as::launch_spmm_wave_rows(crow, col, val, x, y, n, nnz, f, vec4 != 0, s);
   return as::check_launch("spmm_csr");
 }
 

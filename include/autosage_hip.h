@@ -512,9 +512,10 @@ int as_csr_row_softmax_f32(const int64_t* crow, const float* scores,
 /* Bytes of workspace as_csr_attention_f32 needs. */
 size_t as_csr_attention_workspace_bytes(int64_t n, int64_t nnz);
 
-/* Fused out = SpMM(softmax_row(scale * SDDMM(query, key)), value).
- * Replaces csr_attention_forward (autosage/_auto.py:762-780), which runs the
- * three stages separately and has no scale (scale = 1 reproduces it).
+/* out = SpMM(softmax_row(scale * SDDMM(query, key)), value), the three stages
+ * of csr_attention_forward (autosage/_auto.py:762-780) in one call; that one
+ * has no scale (scale = 1 reproduces it).
+ * The first nnz floats of the workspace hold the probabilities afterwards.
  * Bit-identical to as_sddmm_csr_f32 -> as_csr_row_softmax_f32 ->
  * as_spmm_csr_f32 when scale is 1 or a power of two. */
 int as_csr_attention_f32(const int64_t* crow, const int64_t* col,
