@@ -374,7 +374,8 @@ constexpr int64_t kHubBlocksMax = 65536;
 // takes float32 only, csrc/sddmm_csr_op.cu:94; its scheduler runs the
 // gather-dot baseline, autosage/_auto.py:575-581).
 //
-// Vector lanes (F a multiple of 8 up to 512, 16-byte aligned rows): a lane
+// Vector lanes (F a multiple of 8 up to 512, 16-byte aligned rows; by blocks
+// of edges any F from 8 to 512): a lane
 // holds 8 consecutive features, chunk j + G·m of the row for m < MB; G lanes
 // per edge (the power of two covering F/8, at most 32), 64/G edges per
 // gather instruction.  The query row is converted to fp64 once per row and
@@ -590,18 +591,18 @@ void launch_sddmm16_v(const Sddmm16Args& a, dim3 grid, dim3 block, int64_t hub_t
 
 // Lanes per edge G and chunks per lane MB for F features (vector lanes), or
 // G = 0 for element lanes.
-inline void sddmm16_shape(const Sddmm16Args& a, int& g, int& mb) {
+inline void sddmm16_lanes(int64_t f, int& g, int& mb) {
   g = 0;
   mb = 1;
-  if (a.f % 8 != 0 || a.f > 512 || !aligned(a.q, 16) || !aligned(a.k, 16)) return;
-  const int64_t chunks = a.f / 8;
-  if (chunks > 32) {
-    g = 32;
-    mb = 2;
-    return;
-  }
+  if (f < 8 || f > 512) return;
+  const int64_t chunks = (f + 7) / 8;
   g = 1;
-  while (g < chunks) g <<= 1;
+  while (g < chunks && g < 32) g <<= 1;
+  mb = chunks > 32 ? 2 : 1;
+}
+// The split schedule's: element lanes for ragged rows.
+inline void sddmm16_shape(const Sddmm16Args& a, int& g, int& mb) {
+  sddmm16_lanes(a.f % 8 == 0 && aligned(a.q, 16) && aligned(a.k, 16) ? a.f : 0, g, mb);
 }
 
 template <typename T>
@@ -704,11 +705,60 @@ __device__ __forceinline__ const char* chunk_at(const char* base, int row, uint3
   }
 }
 
+// Ragged rows (RAG: F % 8 != 0, or rows that are not 16-byte aligned; F >= 8):
+// the same lanes with loads aligned to an element, the row's last chunk read
+// at F - 8.  The features it shares with the chunk before are cleared on both
+// sides (0 * 0 adds nothing to a sum, which starts at +0).  One wave per edge
+// with a 2-byte lane a feature, us before -> after: 200k rows, 3.2M edges bf16
+// F = 47 434 -> 88, F = 100 491 -> 113; 1M rows, 16M edges F = 47 1985 -> 536,
+// F = 100 2302 -> 783 (F = 48 457, F = 104 760).
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+template <bool RAG>
+__device__ __forceinline__ RawVec<16> load_chunk16(const char* p) {
+  if constexpr (!RAG) {
+    return load_raw<16>(p);
+  } else {
+    const u32x4_a2 v = *reinterpret_cast<const u32x4_a2*>(p);
+    return RawVec<16>{{v[0], v[1], v[2], v[3]}};
+  }
+}
+
+// A lane's chunks j + G·m of rows of F features.
+template <int G, int MB, bool RAG>
+struct Chunks16 {
+  int chunks;
+  uint32_t off[MB];
+  uint32_t mask[RAG ? MB : 1][4];
+  __device__ __forceinline__ Chunks16(int64_t F, int j) {
+    chunks = static_cast<int>(RAG ? (F + 7) / 8 : F / 8);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int c = j + G * m;
+      off[m] = static_cast<uint32_t>((c < chunks ? c : 0) * 16);
+      if constexpr (RAG) {
+        const int dup = c == chunks - 1 ? static_cast<int>(chunks * 8 - F) : 0;
+        off[m] -= static_cast<uint32_t>(dup * 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mask[m][i] = 2 * i + 1 < dup ? 0u : (2 * i < dup ? 0xffff0000u : ~0u);
+      }
+    }
+  }
+  template <typename T>
+  __device__ __forceinline__ double get(const RawVec<16>& v, int m, int p) const {
+    if constexpr (RAG) {
+      const uint32_t w = v.w[p >> 1] & mask[m][p >> 1];
+      return static_cast<double>(Elem<T>::get(&w, p & 1));
+    } else {
+      return static_cast<double>(Elem<T>::get(v.w, p));
+    }
+  }
+};
+
 // The dot products of one block of cnt <= 64 edges starting at edge b,
 // vector lanes: lane j of lane group g holds chunks j + G·m of the edge's
 // query and key rows.  my_c / my_row: lane i holds the column / row of edge
 // b + i.
-template <typename T, int G, int MB, bool OFF32>
+template <typename T, int G, int MB, bool OFF32, bool RAG>
 __device__ __forceinline__ void edge_block16_vec(const char* __restrict__ kb, const char* __restrict__ qb,
                                                  uint16_t* __restrict__ out, int64_t F, int64_t b, int cnt, int my_c,
                                                  int my_row) {
@@ -721,11 +771,8 @@ __device__ __forceinline__ void edge_block16_vec(const char* __restrict__ kb, co
   const int lane = lane_id();
   const int g = lane / G;
   const int j = lane % G;
-  const int64_t chunks = F / 8;
+  const Chunks16<G, MB, RAG> lanes(F, j);
   const uint32_t row_bytes = static_cast<uint32_t>(F * sizeof(T));
-  uint32_t lane_off[MB];
-#pragma unroll
-  for (int m = 0; m < MB; ++m) lane_off[m] = static_cast<uint32_t>((j + G * m < chunks ? j + G * m : 0) * 16);
   for (int u0 = 0; u0 < cnt; u0 += kSub) {
     RawVec<16> kv[UE][MB];
     RawVec<16> qv[UE][MB];
@@ -737,8 +784,8 @@ __device__ __forceinline__ void edge_block16_vec(const char* __restrict__ kb, co
         const int rw = __builtin_amdgcn_ds_bpermute(addr, my_row);
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
-          kv[u][m] = load_raw<16>(chunk_at<OFF32>(kb, c, row_bytes, lane_off[m]));
-          qv[u][m] = load_raw<16>(chunk_at<OFF32>(qb, rw, row_bytes, lane_off[m]));
+          kv[u][m] = load_chunk16<RAG>(chunk_at<OFF32>(kb, c, row_bytes, lanes.off[m]));
+          qv[u][m] = load_chunk16<RAG>(chunk_at<OFF32>(qb, rw, row_bytes, lanes.off[m]));
         }
       }
     }
@@ -748,11 +795,10 @@ __device__ __forceinline__ void edge_block16_vec(const char* __restrict__ kb, co
         double acc = 0.0;
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
-          if (j + G * m < chunks) {
+          if (j + G * m < lanes.chunks) {
 #pragma unroll
             for (int p = 0; p < 8; ++p)
-              acc = __builtin_fma(static_cast<double>(Elem<T>::get(qv[u][m].w, p)),
-                                  static_cast<double>(Elem<T>::get(kv[u][m].w, p)), acc);
+              acc = __builtin_fma(lanes.template get<T>(qv[u][m], m, p), lanes.template get<T>(kv[u][m], m, p), acc);
           }
         }
 #pragma unroll
@@ -767,7 +813,7 @@ __device__ __forceinline__ void edge_block16_vec(const char* __restrict__ kb, co
 // A wave whose edges [b0, b1) all lie in row `row` (long rows): the lane's
 // query chunks are loaded once and the blocks need no row lookup.  The same
 // products, sums and butterfly.
-template <typename T, int G, int MB, bool OFF32>
+template <typename T, int G, int MB, bool OFF32, bool RAG>
 __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ col, const char* __restrict__ kb,
                                                     const char* __restrict__ qb, uint16_t* __restrict__ out,
                                                     int64_t F, int64_t b0, int64_t b1, int row) {
@@ -778,15 +824,11 @@ __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ 
   const int lane = lane_id();
   const int g = lane / G;
   const int j = lane % G;
-  const int64_t chunks = F / 8;
+  const Chunks16<G, MB, RAG> lanes(F, j);
   const uint32_t row_bytes = static_cast<uint32_t>(F * sizeof(T));
-  uint32_t lane_off[MB];
   RawVec<16> q[MB];
 #pragma unroll
-  for (int m = 0; m < MB; ++m) {
-    lane_off[m] = static_cast<uint32_t>((j + G * m < chunks ? j + G * m : 0) * 16);
-    q[m] = load_raw<16>(chunk_at<OFF32>(qb, row, row_bytes, lane_off[m]));
-  }
+  for (int m = 0; m < MB; ++m) q[m] = load_chunk16<RAG>(chunk_at<OFF32>(qb, row, row_bytes, lanes.off[m]));
   int next_c = b0 + lane < b1 ? static_cast<int>(col[b0 + lane]) : 0;
   for (int64_t b = b0; b < b1; b += kWave) {
     const int cnt = b1 - b < kWave ? static_cast<int>(b1 - b) : kWave;
@@ -799,7 +841,7 @@ __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ 
         if (u0 + u * NG < cnt) {
           const int c = __builtin_amdgcn_ds_bpermute((u0 + u * NG + g) * 4, my_c);
 #pragma unroll
-          for (int m = 0; m < MB; ++m) kv[u][m] = load_raw<16>(chunk_at<OFF32>(kb, c, row_bytes, lane_off[m]));
+          for (int m = 0; m < MB; ++m) kv[u][m] = load_chunk16<RAG>(chunk_at<OFF32>(kb, c, row_bytes, lanes.off[m]));
         }
       }
 #pragma unroll
@@ -808,11 +850,10 @@ __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ 
           double acc = 0.0;
 #pragma unroll
           for (int m = 0; m < MB; ++m) {
-            if (j + G * m < chunks) {
+            if (j + G * m < lanes.chunks) {
 #pragma unroll
               for (int p = 0; p < 8; ++p)
-                acc = __builtin_fma(static_cast<double>(Elem<T>::get(q[m].w, p)),
-                                    static_cast<double>(Elem<T>::get(kv[u][m].w, p)), acc);
+                acc = __builtin_fma(lanes.template get<T>(q[m], m, p), lanes.template get<T>(kv[u][m], m, p), acc);
             }
           }
 #pragma unroll
@@ -825,7 +866,7 @@ __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ 
   }
 }
 
-template <typename T, int G, int MB, bool VEC, bool OFF32>
+template <typename T, int G, int MB, bool VEC, bool OFF32, bool RAG>
 __global__ __launch_bounds__(kEdgeWaves * kWave) __attribute__((amdgpu_waves_per_eu(8))) void sddmm16_edges_kernel(
     const int64_t* __restrict__ crow, const int64_t* __restrict__ col, const T* __restrict__ query,
     const T* __restrict__ key, uint16_t* __restrict__ out, int64_t n, int64_t nnz, int64_t F,
@@ -840,7 +881,7 @@ __global__ __launch_bounds__(kEdgeWaves * kWave) __attribute__((amdgpu_waves_per
   const char* __restrict__ qb = reinterpret_cast<const char*>(query);
   if constexpr (VEC) {
     if (uniform_i64(crow[r + 1]) >= b1) {  // every edge of the wave is in row r
-      one_row_edges16_vec<T, G, MB, OFF32>(col, kb, qb, out, F, b0, b1, static_cast<int>(r));
+      one_row_edges16_vec<T, G, MB, OFF32, RAG>(col, kb, qb, out, F, b0, b1, static_cast<int>(r));
       return;
     }
   }
@@ -852,7 +893,7 @@ __global__ __launch_bounds__(kEdgeWaves * kWave) __attribute__((amdgpu_waves_per
     const int my_row = block_edge_rows(crow, n, b, cnt, r);
     r = __builtin_amdgcn_readlane(my_row, cnt - 1);
     if constexpr (VEC) {
-      edge_block16_vec<T, G, MB, OFF32>(kb, qb, out, F, b, cnt, my_c, my_row);
+      edge_block16_vec<T, G, MB, OFF32, RAG>(kb, qb, out, F, b, cnt, my_c, my_row);
     } else {
       // element lanes: lane l adds features l, l + 64, ... of each edge in
       // turn (the order of dots16_scalar)
@@ -878,21 +919,24 @@ void launch_sddmm16_edges(const Sddmm16Args& a, int64_t nnz, int32_t* wave_rows,
   hipLaunchKernelGGL(edge_wave_rows_kernel, dim3(static_cast<unsigned>((waves + 255) / 256)), dim3(256), 0, s,
                      a.crow, a.n, waves, wave_rows);
   int g, mb;
-  sddmm16_shape(a, g, mb);
+  const bool ragged = a.f % 8 != 0 || !aligned(a.q, 16) || !aligned(a.k, 16);
+  sddmm16_lanes(a.f, g, mb);
   const bool off32 = sddmm16_off32(a);
   const int64_t blocks = (waves + kEdgeWaves - 1) / kEdgeWaves;
   for (int64_t b0 = 0; b0 < blocks; b0 += kMaxBlocksPerLaunch) {
     const int64_t nb = blocks - b0 < kMaxBlocksPerLaunch ? blocks - b0 : kMaxBlocksPerLaunch;
     const dim3 grid(static_cast<unsigned>(nb));
     const dim3 block(kEdgeWaves * kWave);
-#define AS_E16(G, MB, VEC, OFF)                                                                              \
-  hipLaunchKernelGGL((sddmm16_edges_kernel<T, G, MB, VEC, OFF>), grid, block, 0, s, a.crow, a.col,           \
+#define AS_E16(G, MB, VEC, OFF, RAG)                                                                         \
+  hipLaunchKernelGGL((sddmm16_edges_kernel<T, G, MB, VEC, OFF, RAG>), grid, block, 0, s, a.crow, a.col,           \
                      static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<uint16_t*>(a.out), a.n, \
                      nnz, a.f, wave_rows, waves, b0 * kEdgeWaves)
-#define AS_E16_V(G, MB)                  \
-  do {                                   \
-    if (off32) AS_E16(G, MB, true, true); \
-    else AS_E16(G, MB, true, false);      \
+#define AS_E16_V(G, MB)                                    \
+  do {                                                     \
+    if (ragged && off32) AS_E16(G, MB, true, true, true);   \
+    else if (ragged) AS_E16(G, MB, true, false, true);      \
+    else if (off32) AS_E16(G, MB, true, true, false);       \
+    else AS_E16(G, MB, true, false, false);                 \
   } while (0)
     if (mb == 2) {
       AS_E16_V(32, 2);
@@ -904,7 +948,7 @@ void launch_sddmm16_edges(const Sddmm16Args& a, int64_t nnz, int32_t* wave_rows,
         case 8: AS_E16_V(8, 1); break;
         case 16: AS_E16_V(16, 1); break;
         case 32: AS_E16_V(32, 1); break;
-        default: AS_E16(64, 1, false, false); break;
+        default: AS_E16(64, 1, false, false, false); break;
       }
     }
 #undef AS_E16_V
