@@ -100,5 +100,17 @@ __device__ __forceinline__ RawVec<BYTES> load_raw(const char* p) {
   return r;
 }
 
+// 16 bytes of 16-bit elements; ANY: aligned to an element only.
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+template <bool ANY>
+__device__ __forceinline__ RawVec<16> load_raw16(const char* p) {
+  if constexpr (!ANY) {
+    return load_raw<16>(p);
+  } else {
+    const u32x4_a2 v = *reinterpret_cast<const u32x4_a2*>(p);
+    return RawVec<16>{{v[0], v[1], v[2], v[3]}};
+  }
+}
+
 }  // namespace
 }  // namespace as

@@ -712,17 +712,6 @@ __device__ __forceinline__ const char* chunk_at(const char* base, int row, uint3
 // with a 2-byte lane a feature, us before -> after: 200k rows, 3.2M edges bf16
 // F = 47 434 -> 88, F = 100 491 -> 113; 1M rows, 16M edges F = 47 1985 -> 536,
 // F = 100 2302 -> 783 (F = 48 457, F = 104 760).
-typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-template <bool RAG>
-__device__ __forceinline__ RawVec<16> load_chunk16(const char* p) {
-  if constexpr (!RAG) {
-    return load_raw<16>(p);
-  } else {
-    const u32x4_a2 v = *reinterpret_cast<const u32x4_a2*>(p);
-    return RawVec<16>{{v[0], v[1], v[2], v[3]}};
-  }
-}
-
 // A lane's chunks j + G·m of rows of F features.
 template <int G, int MB, bool RAG>
 struct Chunks16 {
@@ -784,8 +773,8 @@ __device__ __forceinline__ void edge_block16_vec(const char* __restrict__ kb, co
         const int rw = __builtin_amdgcn_ds_bpermute(addr, my_row);
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
-          kv[u][m] = load_chunk16<RAG>(chunk_at<OFF32>(kb, c, row_bytes, lanes.off[m]));
-          qv[u][m] = load_chunk16<RAG>(chunk_at<OFF32>(qb, rw, row_bytes, lanes.off[m]));
+          kv[u][m] = load_raw16<RAG>(chunk_at<OFF32>(kb, c, row_bytes, lanes.off[m]));
+          qv[u][m] = load_raw16<RAG>(chunk_at<OFF32>(qb, rw, row_bytes, lanes.off[m]));
         }
       }
     }
@@ -828,7 +817,7 @@ __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ 
   const uint32_t row_bytes = static_cast<uint32_t>(F * sizeof(T));
   RawVec<16> q[MB];
 #pragma unroll
-  for (int m = 0; m < MB; ++m) q[m] = load_chunk16<RAG>(chunk_at<OFF32>(qb, row, row_bytes, lanes.off[m]));
+  for (int m = 0; m < MB; ++m) q[m] = load_raw16<RAG>(chunk_at<OFF32>(qb, row, row_bytes, lanes.off[m]));
   int next_c = b0 + lane < b1 ? static_cast<int>(col[b0 + lane]) : 0;
   for (int64_t b = b0; b < b1; b += kWave) {
     const int cnt = b1 - b < kWave ? static_cast<int>(b1 - b) : kWave;
@@ -841,7 +830,7 @@ __device__ __forceinline__ void one_row_edges16_vec(const int64_t* __restrict__ 
         if (u0 + u * NG < cnt) {
           const int c = __builtin_amdgcn_ds_bpermute((u0 + u * NG + g) * 4, my_c);
 #pragma unroll
-          for (int m = 0; m < MB; ++m) kv[u][m] = load_chunk16<RAG>(chunk_at<OFF32>(kb, c, row_bytes, lanes.off[m]));
+          for (int m = 0; m < MB; ++m) kv[u][m] = load_raw16<RAG>(chunk_at<OFF32>(kb, c, row_bytes, lanes.off[m]));
         }
       }
 #pragma unroll

@@ -188,6 +188,14 @@ __device__ __forceinline__ void slice_row(const int64_t* __restrict__ col, const
   }
 }
 
+// The first of a lane's P features: as given, or (RAG: rows of F >= P features
+// at any alignment) at most F - P, so that the last lane's overlap the lane
+// before; both sum and store the same bits.
+template <bool RAG, int P>
+__device__ __forceinline__ int64_t lane_features(int64_t f, int64_t F) {
+  return RAG && f > F - P ? F - P : f;
+}
+
 // Wide form of slice_row for F a multiple of P and 16-byte aligned X: G lanes
 // per edge, each lane owning P = 16 / sizeof(T) consecutive features (one
 // 16-byte load: 4 fp32 or 8 bf16 / fp16), so that one gather instruction
@@ -196,7 +204,7 @@ __device__ __forceinline__ void slice_row(const int64_t* __restrict__ col, const
 // takes edges j + k, j + EPI + k, ... and keeps its own fp64 sums; the groups
 // are added at the end in a fixed butterfly order.  One call covers the
 // feature tile [f0, f0 + P·G).
-template <typename T, int G, bool HAS_VAL, int U, typename OutT>
+template <typename T, int G, bool HAS_VAL, int U, bool RAG = false, typename OutT>
 __device__ __forceinline__ void slice_row_wide(const int64_t* __restrict__ col, const T* __restrict__ val,
                                                const T* __restrict__ x, OutT* __restrict__ out, int64_t F,
                                                int64_t rs, int64_t re, int64_t f0) {
@@ -209,9 +217,10 @@ __device__ __forceinline__ void slice_row_wide(const int64_t* __restrict__ col, 
   rs = uniform_i64(rs);
   re = uniform_i64(re);
   {
-    const int64_t fl = f0 + P * static_cast<int64_t>(gl);
-    const bool active = fl < F;
-    const uint32_t lane_bytes = static_cast<uint32_t>((active ? fl : f0) * sizeof(T));
+    const int64_t first = f0 + P * static_cast<int64_t>(gl);
+    const bool active = first < F;
+    const int64_t fl = lane_features<RAG, P>(active ? first : f0, F);
+    const uint32_t lane_bytes = static_cast<uint32_t>(fl * sizeof(T));
     double acc[P];
 #pragma unroll
     for (int v = 0; v < P; ++v) acc[v] = 0.0;
@@ -251,7 +260,7 @@ __device__ __forceinline__ void slice_row_wide(const int64_t* __restrict__ col, 
               w[u] = grp == k ? wk : w[u];
             }
           }
-          xv[u] = load_raw<16>(xb + row_offset(c, F) * sizeof(T) + lane_bytes);
+          xv[u] = load_raw16<RAG>(xb + row_offset(c, F) * sizeof(T) + lane_bytes);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -295,7 +304,7 @@ __device__ __forceinline__ void slice_row_wide(const int64_t* __restrict__ col, 
 // On the 115M-edge skewed benchmark graph at F = 64 fp32 this takes the call
 // from 2.18 to 2.00 ms; with 32-lane groups (2 edges per gather) the same
 // changes cost about 1 %, so those keep slice_row_wide.
-template <typename T, int G, bool HAS_VAL, int U, bool OFF32, typename OutT>
+template <typename T, int G, bool HAS_VAL, int U, bool OFF32, bool RAG, typename OutT>
 __device__ __forceinline__ void slice_row_wide_bpermute(const int64_t* __restrict__ col,
                                                         const T* __restrict__ val, const T* __restrict__ x,
                                                         OutT* __restrict__ out, int64_t F, int64_t rs, int64_t re,
@@ -309,9 +318,10 @@ __device__ __forceinline__ void slice_row_wide_bpermute(const int64_t* __restric
   const int gl = lane % G;
   rs = uniform_i64(rs);
   re = uniform_i64(re);
-  const int64_t fl = f0 + P * static_cast<int64_t>(gl);
-  const bool active = fl < F;
-  const uint32_t lane_bytes = static_cast<uint32_t>((active ? fl : f0) * sizeof(T));
+  const int64_t first = f0 + P * static_cast<int64_t>(gl);
+  const bool active = first < F;
+  const int64_t fl = lane_features<RAG, P>(active ? first : f0, F);
+  const uint32_t lane_bytes = static_cast<uint32_t>(fl * sizeof(T));
   const uint32_t row_bytes = static_cast<uint32_t>(F * sizeof(T));
   const char* __restrict__ xb = reinterpret_cast<const char*>(x);
   double acc[P];
@@ -330,9 +340,9 @@ __device__ __forceinline__ void slice_row_wide_bpermute(const int64_t* __restric
     const int c = __builtin_amdgcn_ds_bpermute(addr, my_col);
     if constexpr (HAS_VAL) w = __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(my_w)));
     if constexpr (OFF32) {
-      return load_raw<16>(xb + (__umul24(static_cast<uint32_t>(c), row_bytes) + lane_bytes));
+      return load_raw16<RAG>(xb + (__umul24(static_cast<uint32_t>(c), row_bytes) + lane_bytes));
     } else {
-      return load_raw<16>(xb + row_offset(c, F) * sizeof(T) + lane_bytes);
+      return load_raw16<RAG>(xb + row_offset(c, F) * sizeof(T) + lane_bytes);
     }
   };
   auto add = [&](const RawVec<16>& xv, float w) {
@@ -393,7 +403,7 @@ __device__ __forceinline__ void slice_row_wide_bpermute(const int64_t* __restric
 #define AS_COLSLICE_WIDE_U_16 2
 #endif
 
-template <typename T, int G, bool HAS_VAL, bool OFF32, typename OutT>
+template <typename T, int G, bool HAS_VAL, bool OFF32, bool RAG = false, typename OutT>
 __device__ __forceinline__ void slice_wide(const int64_t* __restrict__ col, const T* __restrict__ val,
                                            const T* __restrict__ x, OutT* __restrict__ out, int64_t F, int64_t rs,
                                            int64_t re, int64_t f0) {
@@ -401,9 +411,9 @@ __device__ __forceinline__ void slice_wide(const int64_t* __restrict__ col, cons
     // 16-bit lanes carry 8 fp64 sums: 2 gathers per batch keep the wave
     // within 64 VGPRs (8 waves per SIMD)
     constexpr int U = sizeof(T) == 2 ? AS_COLSLICE_WIDE_U_16 : AS_COLSLICE_WIDE_U;
-    slice_row_wide_bpermute<T, G, HAS_VAL, U, OFF32>(col, val, x, out, F, rs, re, f0);
+    slice_row_wide_bpermute<T, G, HAS_VAL, U, OFF32, RAG>(col, val, x, out, F, rs, re, f0);
   } else {
-    slice_row_wide<T, G, HAS_VAL, AS_COLSLICE_WIDE_U>(col, val, x, out, F, rs, re, f0);
+    slice_row_wide<T, G, HAS_VAL, AS_COLSLICE_WIDE_U, RAG>(col, val, x, out, F, rs, re, f0);
   }
 }
 
@@ -1054,7 +1064,14 @@ enum Slicing { kSliceColumns = 0, kSliceEdges = 1 };
 // tile t sums rows w, w + W, ... whole (the short-row forms above, rounded
 // once into Y).  For small graphs, where the slice points, the binning and the
 // chunk launches of the sliced schedule cost more than the product.
-template <typename T, int V, bool HAS_VAL, bool OFF32>
+// RAG: F % 8 != 0 or X not 16-byte aligned and more than 64 features, on the
+// same 16-byte lanes (element alignment is enough).  Those rows on 2-byte lanes
+// against this, bf16 us: 200k rows, 3.2M edges F = 100 312 / 176, F = 199 609 / 333;
+// 1M rows, 16M edges F = 100 1012 / 703, F = 199 2319 / 1267.  Up to 64 features a
+// wave covers the row with a 2-byte lane a feature in one step and is the faster
+// one where rows are short (40k rows of 10 edges F = 15 19 / 26, F = 47 22 / 27; 1M rows,
+// 16M edges F = 31 506 / 549, F = 63 590 / 570).
+template <typename T, int V, bool HAS_VAL, bool OFF32, bool RAG>
 __global__ __launch_bounds__(kBlock) void rows16_kernel(const int64_t* __restrict__ crow,
                                                         const int64_t* __restrict__ col, const T* __restrict__ val,
                                                         const T* __restrict__ x, T* __restrict__ y, int64_t n,
@@ -1067,7 +1084,7 @@ __global__ __launch_bounds__(kBlock) void rows16_kernel(const int64_t* __restric
     const int64_t rs = uniform_i64(crow[row]);
     const int64_t re = uniform_i64(crow[row + 1]);
     if constexpr (V >= 8) {
-      slice_wide<T, V, HAS_VAL, OFF32>(col, val, x, y + row * F, F, rs, re, tile * kTile);
+      slice_wide<T, V, HAS_VAL, OFF32, RAG>(col, val, x, y + row * F, F, rs, re, tile * kTile);
     } else {
       slice_row<T, V, HAS_VAL, 8>(col, val, x, y + row * F, F, rs, re);
     }
@@ -1079,7 +1096,8 @@ int rows16_run(const int64_t* crow, const int64_t* col, const void* val, const v
                int64_t f, hipStream_t s) {
   constexpr int64_t P = 8;  // 16-bit elements per 16-byte lane
   int v = 1;
-  if (f % P == 0 && aligned(x, 16)) v = f <= 64 ? 8 : (f <= 128 ? 16 : 32);
+  const bool ragged = f % P != 0 || !aligned(x, 16);
+  if (!ragged || f > 64) v = f <= 64 ? 8 : (f <= 128 ? 16 : 32);
   const int64_t tiles = v >= 8 ? (f + P * v - 1) / (P * v) : 1;
   const bool off32 = n <= (int64_t(1) << 24) && f * 2 < (int64_t(1) << 24) && n * f * 2 <= (int64_t(1) << 32);
   int64_t tile_blocks = (n + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -1090,14 +1108,23 @@ int rows16_run(const int64_t* crow, const int64_t* col, const void* val, const v
   const T* vp = static_cast<const T*>(val);
   const T* xp = static_cast<const T*>(x);
   T* yp = static_cast<T*>(y);
-#define AS_ROWS16(V_, O_) \
-  hipLaunchKernelGGL((rows16_kernel<T, V_, HAS_VAL, O_>), grid, dim3(kBlock), 0, s, crow, col, vp, xp, yp, n, f, tile_blocks)
+#define AS_ROWS16(V_, O_, R_)                                                                                 \
+  hipLaunchKernelGGL((rows16_kernel<T, V_, HAS_VAL, O_, R_>), grid, dim3(kBlock), 0, s, crow, col, vp, xp, yp, n, f, \
+                     tile_blocks)
+#define AS_ROWS16_V(V_)                             \
+  do {                                              \
+    if (ragged && off32) AS_ROWS16(V_, true, true);   \
+    else if (ragged) AS_ROWS16(V_, false, true);      \
+    else if (off32) AS_ROWS16(V_, true, false);       \
+    else AS_ROWS16(V_, false, false);                 \
+  } while (0)
   switch (v) {
-    case 32: if (off32) AS_ROWS16(32, true); else AS_ROWS16(32, false); break;
-    case 16: if (off32) AS_ROWS16(16, true); else AS_ROWS16(16, false); break;
-    case 8: if (off32) AS_ROWS16(8, true); else AS_ROWS16(8, false); break;
-    default: AS_ROWS16(1, false); break;
+    case 32: AS_ROWS16_V(32); break;
+    case 16: AS_ROWS16_V(16); break;
+    case 8: if (off32) AS_ROWS16(8, true, false); else AS_ROWS16(8, false, false); break;
+    default: AS_ROWS16(1, false, false); break;
   }
+#undef AS_ROWS16_V
 #undef AS_ROWS16
   return AS_OK;
 }
