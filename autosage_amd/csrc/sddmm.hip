@@ -495,7 +495,7 @@ __device__ __forceinline__ void sddmm16_edges(const int64_t* __restrict__ col, c
   }
 }
 
-// The split schedule of sddmm_scheduled_kernel for 16-bit elements:
+// The split schedule for 16-bit elements:
 // workgroups [0, hub_blocks) stride over the 2048-edge chunks of the rows of
 // degree >= hub_threshold, the rest take the other rows one per wave.
 template <typename T, int G, int MB, bool VEC, bool OFF32>

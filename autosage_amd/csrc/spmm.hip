@@ -10,6 +10,9 @@
 // sequential CPU CSR product, so the result is bit-identical to it whatever
 // the row-to-wave mapping, feature slicing or vector width.
 //
+// The whole graph goes to spmm_groups.hip except where one wave per row is the
+// better form (as_spmm_csr_rows_f32).
+//
 // Row layouts:
 //   wave-row  one wave64 owns a row (or a feature slice of it); lane owns V in
 //             {1,2,4} consecutive features; a pass covers 64·V features.

@@ -388,7 +388,7 @@ size_t as_spmm_rounded_16_workspace_bytes(int64_t n, int64_t f, int64_t sliced_r
 /* The product of as_spmm_csr_rounded_16 (same bits) without slicing: one
  * launch, no workspace, every row summed whole by one wavefront.  For small
  * graphs, where the sliced schedule's set-up costs more than the product;
- * any column order. */
+ * any column order.  F above 64 takes 16-byte lanes at any alignment. */
 int as_spmm_csr_rows_16(const int64_t* crow, const int64_t* col, const void* val,
                         const void* x, void* y, int64_t n, int64_t nnz, int64_t f,
                         int dtype, void* stream);
@@ -430,8 +430,9 @@ size_t as_sddmm_edges_16_workspace_bytes(int64_t nnz);
 /* The SDDMM of as_sddmm_csr_rounded_16 (the same bits) on another schedule:
  * the edges in CSR order in blocks of 64, a few blocks per wavefront,
  * whatever the row lengths, each edge's row found from crow inside the
- * wavefront; no degree split.  Same arguments as as_sddmm_csr_rounded_16
- * without the split settings.  Replaces sddmm_csr (csrc/sddmm_csr_op.cu:108-134)
+ * wavefront; no degree split.  F from 8 to 512 takes 16-byte lanes at any
+ * alignment.  Same arguments as as_sddmm_csr_rounded_16 without the split
+ * settings.  Replaces sddmm_csr (csrc/sddmm_csr_op.cu:108-134)
  * for the 16-bit types the reference leaves to its gather-dot baseline
  * (autosage/_auto.py:575-581). */
 int as_sddmm_csr_edges_16(const int64_t* crow, const int64_t* col,
