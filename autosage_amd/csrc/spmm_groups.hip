@@ -12,7 +12,7 @@
 // wave owns up to 60 consecutive rows and hands the next one to each lane group
 // that finishes; a batch of 8 edges' column indices is loaded one batch ahead.
 //
-// Long rows (at least kSpmmLongRow edges): one chain per feature is a chain of
+// Long rows (at least kSpmmLongRow edges; half of that in small graphs): one chain per feature is a chain of
 // dependent additions, but its gathers need not wait for it.  The first
 // workgroups of the launch each scan a strided share of crow for long rows and
 // take them one after another (per slice of at most 64 features): 3 waves gather
@@ -55,6 +55,7 @@ struct GroupArgs {
   int64_t hub_stride;  // hub workgroups per feature slice (0: no long rows)
   int hub_slices;
   int hub_width;       // features per slice (a multiple of 4, <= 64)
+  int64_t long_row;  // edges from which a workgroup takes a row
 };
 
 // ---- long rows ---------------------------------------------------------------
@@ -273,7 +274,7 @@ __device__ __forceinline__ void hub_block(const GroupArgs& a, int64_t block, Hub
     if (line < lines && row < a.n) {
       const int64_t rs = a.crow[row];
       const int64_t len = a.crow[row + 1] - rs;
-      if (len >= kSpmmLongRow) {
+      if (len >= a.long_row) {
         const int at = atomicAdd(&sh.count, 1);
         sh.first[at] = rs;
         sh.len[at] = len;
@@ -344,7 +345,7 @@ __device__ __forceinline__ void light_groups(const GroupArgs& a, int64_t light) 
       const int64_t re = static_cast<int64_t>(__shfl(static_cast<long long>(ends), i1, kWave));
       if (need) {
         next.row = idx < pool ? row0 + idx : -1;
-        next.hub = a.hub_stride > 0 && re - rs >= kSpmmLongRow;
+        next.hub = a.hub_stride > 0 && re - rs >= a.long_row;
         k = rs;
         end = next.hub ? rs : re;
       }
@@ -454,7 +455,7 @@ void launch_groups(const GroupArgs& a, int64_t light, bool off32, hipStream_t s)
 
 void launch_spmm_groups(const int64_t* crow, const int64_t* col, const float* val, const float* x, float* y, int64_t n,
                         int64_t n_cols, int64_t nnz, int64_t f, hipStream_t s) {
-  GroupArgs a{crow, col, val, x, y, n, nnz, f, 0, 0, 0, 0, 0, 0, 1, 64};
+  GroupArgs a{crow, col, val, x, y, n, nnz, f, 0, 0, 0, 0, 0, 0, 1, 64, kSpmmLongRow};
   a.tiles = static_cast<int>((f + 255) / 256);
   a.tile = static_cast<int>(((f + a.tiles - 1) / a.tiles + 3) / 4 * 4);
   a.lpr = a.tile / 4;
@@ -472,12 +473,19 @@ void launch_spmm_groups(const int64_t* crow, const int64_t* col, const float* va
   int64_t m = n / (static_cast<int64_t>(a.rpw) * 16384);
   m = m < 1 ? 1 : (m > most ? most : m);
   a.pool = static_cast<int>(a.rpw * m < 60 ? a.rpw * m : 60);
-  if (nnz >= kSpmmLongRow) {
+  // graphs of few rows leave the chip idle, so rows that are short elsewhere go to
+  // workgroups too (1000 rows of 30 edges, longest 200, F = 64: 17.4 -> 12.0 us; 2,600
+  // rows of 59, longest 640, F = 16: 22.9 -> 19.1; level at 10,000 rows)
+  a.long_row = n < 8192 ? kSpmmLongRow / 2 : kSpmmLongRow;
+  if (nnz >= a.long_row) {
     const int64_t wide = (f + 63) / 64;
     a.hub_slices = static_cast<int>(nnz * wide <= kNarrowSliceEdges ? (f + 31) / 32 : wide);
     a.hub_width = static_cast<int>(((f + a.hub_slices - 1) / a.hub_slices + 3) / 4 * 4);
     const int64_t want = kHubBlocks / a.hub_slices > 128 ? kHubBlocks / a.hub_slices : 128;
-    const int64_t share = (n + 63) / 64;  // at least 64 rows to scan
+    // at least 16 rows to scan; with 64 a workgroup took the long rows of a small
+    // graph one after the other (5,000 rows of 64 edges, longest 1,200, F = 16:
+    // 43.8 -> 24.4 us; 10,000 of 40, longest 2,000: 41.9 -> 28.5)
+    const int64_t share = (n + 15) / 16;
     a.hub_stride = want < share ? want : share;
   }
   const int64_t waves = (n + a.pool - 1) / a.pool;

@@ -96,3 +96,11 @@ def test_spmm_rows_known_to_be_even(features, long_row):
     got = torch.ops.autosage.spmm_csr(d_crow, d_col, d_val, d_x)
     ref = oracle.spmm_seq(crow, col, val, x)
     assert bitwise_equal(got, ref), mismatch_report(got, ref)
+
+
+@pytest.mark.parametrize("rows", [40, 8191, 8192])
+@pytest.mark.parametrize("features", [16, 100])
+def test_long_rows_start_lower_in_small_graphs(rows, features):
+    crow, col, rng = _graph([127, 128, 129, 254, 255, 256, 257, 600] * 4 + [2] * (rows - 32), rows)
+    x = rng.standard_normal((rows, features)).astype(np.float32)
+    _check(crow, col, None, x)
