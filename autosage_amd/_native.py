@@ -908,9 +908,13 @@ def csr_attention_probs_impl(crow, col, query, key, value, scale=1.0):
     n, fqk = query.shape
     fv = value.size(1)
     nnz = col.numel()
-    if fqk == 0 and nnz > 0 and fv > 0:
-        # all scores are zero: the softmax of each row is uniform
-        probs = csr_row_softmax_impl(crow, torch.zeros(nnz, dtype=query.dtype, device=query.device))
+    if nnz > 0 and (fqk == 0 or fv == 0):
+        # no query and key features: the scores are zero and the softmax of each
+        # row is uniform; no value features: the native call computes nothing
+        scores = sddmm_csr_impl(crow, col, query, key)
+        if fqk > 0:
+            scores.mul_(float(scale))
+        probs = csr_row_softmax_impl(crow, scores)
         return spmm_csr_impl(crow, col, probs, value), probs
     out = torch.empty((n, fv), dtype=value.dtype, device=value.device)
     lib = library()

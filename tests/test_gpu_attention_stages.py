@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+import autosage_amd
 from gpu_common import require_gpu, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -57,6 +58,31 @@ def test_backward_with_the_forwards_probabilities(which):
     assert all(torch.equal(a, w) for a, w in zip(again, want))
     got = torch.autograd.grad(out, wanted, g)
     assert all(torch.equal(a, w) for a, w in zip(got, want))
+
+
+@pytest.mark.parametrize("fqk", [0, 8])
+def test_values_of_no_width_have_zero_gradients(fqk):
+    """Scores and probabilities exist without value features; the gradients of
+    query and key are 0 whatever the memory held before."""
+    rng = np.random.default_rng(3)
+    lengths = np.array([5, 0, 300, 40] * 50)
+    n = lengths.size
+    crow = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    col = rng.integers(0, n, size=int(crow[-1])).astype(np.int64)
+    d_crow, d_col, q, k, v = to_dev(crow, col, *(rng.standard_normal((n, f)).astype(np.float32) for f in (fqk, fqk, 0)))
+    leaves = [q.requires_grad_(True), k.requires_grad_(True)]
+    for call in (lambda: torch.ops.autosage.csr_attention_probs(d_crow, d_col, q, k, v, 0.5),
+                 lambda: autosage_amd.csr_attention_forward(d_crow, d_col, q, k, v, scale=0.5),
+                 lambda: (torch.ops.autosage.csr_attention(d_crow, d_col, q, k, v, 0.5),)):
+        for _ in range(4):  # freed blocks of this size hold NaN
+            torch.full((col.size,), float("nan"), device="cuda")
+        out = call()[0]
+        assert out.shape == (n, 0)
+        for grad in torch.autograd.grad(out, leaves, torch.empty_like(out)):
+            assert grad.shape == (n, fqk) and not grad.any()
+    _, probs = torch.ops.autosage.csr_attention_probs(d_crow, d_col, q, k, v, 0.5)
+    scores = torch.ops.autosage.sddmm_csr(d_crow, d_col, q, k) * 0.5
+    assert torch.equal(probs, torch.ops.autosage.csr_row_softmax(d_crow, scores))
 
 
 def test_attention_without_edges_is_zero():
