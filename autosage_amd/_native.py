@@ -20,6 +20,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import os
+import threading
 from pathlib import Path
 from typing import Optional
 
@@ -29,7 +30,7 @@ from . import _env
 from ._memo import GraphMemo
 
 LIBRARY_NAME = "libautosage_hip.so"
-ABI_VERSION = 10
+ABI_VERSION = 11
 HUB_EXACT = 0
 HUB_SPLIT64 = 1
 # 16-bit feature types of as_spmm_csr_rounded_16 (AS_DTYPE_BF16 / AS_DTYPE_F16)
@@ -51,9 +52,9 @@ _SIGNATURES = {
     "as_spmm_long_row": (_c_i64, []),
     "as_csr_build_workspace_bytes": (_c_size, [_c_i64, _c_i64]),
     "as_csr_from_edges": (
-        _c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
+        _c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "as_csr_transpose": (
-        _c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
+        _c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "as_bin_workspace_bytes": (_c_size, [_c_i64]),
     "as_bin_rows_by_degree": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "as_spmm_split_workspace_bytes": (_c_size, [_c_i64]),
@@ -1355,30 +1356,55 @@ def csr_build_supported(rows: torch.Tensor, cols: torch.Tensor, n: int) -> bool:
             and not torch.cuda.is_current_stream_capturing())
 
 
-def _csr_build(entry, first, second, n: int, edges: int, want_perm: bool):
+_FLAGS = threading.local()
+
+
+def _check_flag() -> int:
+    """The address of this thread's flag in pinned memory: a build has read it
+    before it returns, so the thread's next build can use it again."""
+    flag = getattr(_FLAGS, "flag", None)
+    if flag is None:
+        flag = _FLAGS.flag = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
+    return flag.data_ptr()
+
+
+def _csr_build(entry, first, second, n: int, edges: int, want_perm: bool, check: bool):
+    """((crow, col, perm), whether the check found bad input)."""
     device = first.device
     lib = library()
     ws = _workspace(lib.as_csr_build_workspace_bytes(n, edges), device)
     crow = torch.empty(n + 1, dtype=torch.long, device=device)
     col = torch.empty(edges, dtype=torch.long, device=device)
     perm = torch.empty(edges, dtype=torch.long, device=device) if want_perm else None
+    bad = _check_flag() if check else None
     with _on(device):
-        status = entry(_ptr(first), _ptr(second), n, edges, _ptr(crow), _ptr(col), _ptr(perm), _ptr(ws), ws.numel(),
-                       _stream(device))
+        status = entry(_ptr(first), _ptr(second), n, edges, _ptr(crow), _ptr(col), _ptr(perm), bad, _ptr(ws),
+                       ws.numel(), _stream(device))
     _raise(status, "autosage CSR build")
-    return crow, col, perm
+    return (crow, col, perm), check and ctypes.c_int32.from_address(bad).value != 0
 
 
 def csr_from_edges(rows: torch.Tensor, cols: torch.Tensor, n: int, want_perm: bool = True):
     """(crow, col, perm or None): the CSR of an edge list on the device, the
-    edges in a stable sort by row (see ``csr_build_supported``)."""
-    return _csr_build(library().as_csr_from_edges, rows, cols, int(n), rows.numel(), want_perm)
+    edges in a stable sort by row (see ``csr_build_supported``); an edge whose
+    row is not in [0, n) is left behind the last row."""
+    return _csr_build(library().as_csr_from_edges, rows, cols, int(n), rows.numel(), want_perm, False)[0]
+
+
+def csr_from_edges_checked(rows: torch.Tensor, cols: torch.Tensor, n: int, want_perm: bool = True):
+    """``csr_from_edges``, or None when a row id is not in [0, n)."""
+    built, bad = _csr_build(library().as_csr_from_edges, rows, cols, int(n), rows.numel(), want_perm, True)
+    return None if bad else built
 
 
 def csr_transpose(crow: torch.Tensor, col: torch.Tensor):
     """(crow_t, col_t, perm) of the transposed n x n CSR on the device, per
     column the source rows in ascending order (see ``csr_build_supported``)."""
-    return _csr_build(library().as_csr_transpose, crow, col, crow.numel() - 1, col.numel(), True)
+    built, bad = _csr_build(library().as_csr_transpose, crow, col, crow.numel() - 1, col.numel(), True, True)
+    if bad:
+        raise RuntimeError("malformed CSR graph: a column outside [0, N), or row pointers that descend or hold "
+                           "fewer edges than there are columns")
+    return built
 
 
 def bin_rows_by_degree(crow: torch.Tensor, threshold: int) -> tuple[torch.Tensor, torch.Tensor]:

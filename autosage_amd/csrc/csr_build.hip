@@ -9,7 +9,11 @@
 // that ids below n have (rocPRIM's radix sort; torch sorts 64-bit keys, below a
 // million of them by merging), then one pass that writes the sorted edges' other
 // ends and finds every row's start by a lower bound over the sorted ids.  No
-// host sync and no count of the ids.
+// count of the ids.
+//
+// The input is checked ahead of the sort, so that the host, which has to know
+// the answer before it hands the CSR out, waits for one short kernel while the
+// sort is already queued behind it, and not for the sort.
 //
 // What bounds it: the sort's passes (8 bits each).  us, torch composition (with its
 // host syncs) -> here: 40k nodes, 400k edges CSR 204 -> 50, transpose 322 -> 56; 1M nodes,
@@ -78,11 +82,70 @@ size_t ids_bytes(int64_t edges) { return align_up(static_cast<size_t>(edges > 0 
 // keys, order, the edges' rows (transpose only), the sort's own
 size_t build_bytes(int64_t n, int64_t edges) { return 3 * ids_bytes(edges) + align_up(sort_temp_bytes(n, edges), 256); }
 
-// rows[e] = the row of edge e: a wave per kExpand edges.
+// Sets *bad, host memory: one store by the first lane of a wave that found
+// something wrong, written back at once.
+__device__ __forceinline__ void report_bad(bool wrong, int32_t* bad) {
+  if (__ballot(wrong) != 0 && lane_id() == 0) {
+    *static_cast<volatile int32_t*>(bad) = 1;
+    __threadfence_system();
+  }
+}
+
+// Does an id lie outside [0, n)?
+__global__ __launch_bounds__(kBlock) void check_ids_kernel(const int64_t* __restrict__ ids, int64_t n, int64_t edges,
+                                                           int32_t* bad) {
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kBlock;
+  bool wrong = false;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < edges; i += step)
+    wrong |= ids[i] < 0 || ids[i] >= n;
+  report_bad(wrong, bad);
+}
+
+// When the check's answer is in *bad (pinned host memory; null: no check):
+// after wait(), which every way out of the call passes.
+class CheckDone {
+ public:
+  CheckDone() = default;
+  CheckDone(const CheckDone&) = delete;
+  CheckDone& operator=(const CheckDone&) = delete;
+  ~CheckDone() {
+    wait();
+    if (event_ != nullptr) (void)hipEventDestroy(event_);
+  }
+  // Behind the launch of the check.
+  bool record(hipStream_t s) {
+    recorded_ = hipEventCreateWithFlags(&event_, hipEventDisableTiming) == hipSuccess &&
+                hipEventRecord(event_, s) == hipSuccess;
+    if (!recorded_) (void)hipStreamSynchronize(s);
+    return recorded_;
+  }
+  bool wait() {
+    if (!recorded_) return true;
+    recorded_ = false;
+    return hipEventSynchronize(event_) == hipSuccess;
+  }
+
+ private:
+  hipEvent_t event_ = nullptr;
+  bool recorded_ = false;
+};
+
+// rows[e] = the row of edge e: a wave per kExpand edges.  With bad, also: does
+// a column lie outside [0, n), do the row pointers descend or hold fewer than
+// `edges` edges?  (The rows are checked by all threads in turn.)
 constexpr int64_t kExpand = 4 * kWave;
-__global__ __launch_bounds__(kBlock) void edge_rows_kernel(const int64_t* __restrict__ crow, int64_t n, int64_t edges,
-                                                           int32_t* __restrict__ rows) {
+__global__ __launch_bounds__(kBlock) void edge_rows_kernel(const int64_t* __restrict__ crow,
+                                                           const int64_t* __restrict__ col, int64_t n, int64_t edges,
+                                                           int32_t* __restrict__ rows, int32_t* bad) {
   const int64_t w = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + wave_in_block();
+  if (bad != nullptr) {
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    bool wrong = first == 0 && crow[n] - crow[0] < edges;
+    for (int64_t r = first; r < n; r += static_cast<int64_t>(gridDim.x) * kBlock) wrong |= crow[r + 1] < crow[r];
+    for (int64_t e = w * kExpand + lane_id(); e < edges && e < (w + 1) * kExpand; e += kWave)
+      wrong |= col[e] < 0 || col[e] >= n;
+    report_bad(wrong, bad);
+  }
   const int64_t b0 = uniform_i64(w * kExpand);
   if (b0 >= edges) return;
   const int64_t b1 = uniform_i64(b0 + kExpand < edges ? b0 + kExpand : edges);
@@ -161,38 +224,53 @@ size_t as_csr_build_workspace_bytes(int64_t n, int64_t edges) {
 }
 
 int as_csr_from_edges(const int64_t* rows, const int64_t* cols, int64_t n, int64_t edges, int64_t* crow, int64_t* col,
-                      int64_t* perm, void* workspace, size_t workspace_bytes, void* stream) {
+                      int64_t* perm, int32_t* bad, void* workspace, size_t workspace_bytes, void* stream) {
   as::clear_error();
   int st = as::validate_build(rows, cols, n, edges, crow, col, workspace, workspace_bytes);
   if (st != AS_OK) return st;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  as::CheckDone check;
+  if (bad != nullptr) {
+    *bad = 0;
+    const int64_t blocks = (edges + 4 * as::kBlock - 1) / (4 * as::kBlock);
+    hipLaunchKernelGGL(as::check_ids_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)),
+                       dim3(as::kBlock), 0, s, rows, n, edges, bad);
+    if (!check.record(s)) return as::fail(AS_ERR_LAUNCH, "checking the edges failed");
+  }
   char* ws = static_cast<char*>(workspace);
   uint32_t* keys = reinterpret_cast<uint32_t*>(ws);
   uint32_t* order = reinterpret_cast<uint32_t*>(ws + as::ids_bytes(edges));
   size_t temp = workspace_bytes - 3 * as::ids_bytes(edges);
   if (as::sort_ids(ws + 3 * as::ids_bytes(edges), temp, rows, n, edges, keys, order, s) != hipSuccess)
     return as::fail(AS_ERR_LAUNCH, "sorting the edges failed");
-  return as::launch_sorted_edges<int64_t>(keys, order, cols, n, edges, crow, col, perm, s);
+  st = as::launch_sorted_edges<int64_t>(keys, order, cols, n, edges, crow, col, perm, s);
+  if (!check.wait()) return as::fail(AS_ERR_LAUNCH, "checking the edges failed");
+  return st;
 }
 
 int as_csr_transpose(const int64_t* crow, const int64_t* col, int64_t n, int64_t nnz, int64_t* crow_t, int64_t* col_t,
-                     int64_t* perm, void* workspace, size_t workspace_bytes, void* stream) {
+                     int64_t* perm, int32_t* bad, void* workspace, size_t workspace_bytes, void* stream) {
   as::clear_error();
   int st = as::validate_build(crow, col, n, nnz, crow_t, col_t, workspace, workspace_bytes);
   if (st != AS_OK) return st;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  as::CheckDone check;
   char* ws = static_cast<char*>(workspace);
   uint32_t* keys = reinterpret_cast<uint32_t*>(ws);
   uint32_t* order = reinterpret_cast<uint32_t*>(ws + as::ids_bytes(nnz));
   int32_t* rows = reinterpret_cast<int32_t*>(ws + 2 * as::ids_bytes(nnz));
+  if (bad != nullptr) *bad = 0;
   const int64_t waves = (nnz + as::kExpand - 1) / as::kExpand;
   hipLaunchKernelGGL(as::edge_rows_kernel,
                      dim3(static_cast<unsigned>((waves + as::kWavesPerBlock - 1) / as::kWavesPerBlock)),
-                     dim3(as::kBlock), 0, s, crow, n, nnz, rows);
+                     dim3(as::kBlock), 0, s, crow, col, n, nnz, rows, bad);
+  if (bad != nullptr && !check.record(s)) return as::fail(AS_ERR_LAUNCH, "checking the graph failed");
   size_t temp = workspace_bytes - 3 * as::ids_bytes(nnz);
   if (as::sort_ids(ws + 3 * as::ids_bytes(nnz), temp, col, n, nnz, keys, order, s) != hipSuccess)
     return as::fail(AS_ERR_LAUNCH, "sorting the edges failed");
-  return as::launch_sorted_edges<int32_t>(keys, order, rows, n, nnz, crow_t, col_t, perm, s);
+  st = as::launch_sorted_edges<int32_t>(keys, order, rows, n, nnz, crow_t, col_t, perm, s);
+  if (!check.wait()) return as::fail(AS_ERR_LAUNCH, "checking the graph failed");
+  return st;
 }
 
 }  // extern "C"

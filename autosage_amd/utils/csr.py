@@ -34,9 +34,17 @@ def _native_csr(rows: torch.Tensor, cols: torch.Tensor, num_nodes: int, want_ord
     from ..ops import load_native
 
     load_native()
-    if not isinstance(num_nodes, int) or not _native.csr_build_supported(rows.contiguous(), cols.contiguous(), num_nodes):
+    rows_c, cols_c = rows.contiguous(), cols.contiguous()
+    if not isinstance(num_nodes, int) or not _native.csr_build_supported(rows_c, cols_c, num_nodes):
         return None, None, None
-    return _native.csr_from_edges(rows.contiguous(), cols.contiguous(), num_nodes, want_order)
+    built = _native.csr_from_edges_checked(rows_c, cols_c, num_nodes, want_order)
+    if built is None:
+        # an id outside [0, num_nodes): refused as on the CPU, but for -1, which
+        # the torch steps count ahead of the first row
+        if bool(((rows < -1) | (rows >= num_nodes)).any()):
+            raise IndexError("edge_index holds a node id outside [0, num_nodes)")
+        return None, None, None
+    return built
 
 
 def csr_with_edge_order(

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define AS_ABI_VERSION 10
+#define AS_ABI_VERSION 11
 
 typedef enum as_status {
   AS_OK = 0,
@@ -98,18 +98,23 @@ size_t as_csr_build_workspace_bytes(int64_t n, int64_t edges);
  * outputs of edge_index_to_csr (autosage/utils/csr.py:6-26), bit for bit;
  * crow int64[n + 1], col int64[edges], perm int64[edges] or null.  An edge
  * whose row id lies outside [0, n) is left behind the last row (crow[n]).
- * No host sync; not for stream capture (the sort may record memsets). */
+ * bad (pinned host memory, or null): set to 1 if there is such an edge, else
+ * to 0; the call then waits for the pass that looks for it, queued ahead of
+ * the sort, and without bad it does not wait.  Not for stream capture (the
+ * sort may record memsets). */
 int as_csr_from_edges(const int64_t* rows, const int64_t* cols, int64_t n,
                       int64_t edges, int64_t* crow, int64_t* col, int64_t* perm,
-                      void* workspace, size_t workspace_bytes, void* stream);
+                      int32_t* bad, void* workspace, size_t workspace_bytes,
+                      void* stream);
 
 /* The transpose of an n x n CSR (no reference counterpart): per column the
- * source rows in ascending order, col_t[k] = row of edge perm[k].  As
- * as_csr_from_edges otherwise. */
+ * source rows in ascending order, col_t[k] = row of edge perm[k].  bad is set
+ * for a column outside [0, n), descending row pointers and ones that hold
+ * fewer than nnz edges.  As as_csr_from_edges otherwise. */
 int as_csr_transpose(const int64_t* crow, const int64_t* col, int64_t n,
                      int64_t nnz, int64_t* crow_t, int64_t* col_t,
-                     int64_t* perm, void* workspace, size_t workspace_bytes,
-                     void* stream);
+                     int64_t* perm, int32_t* bad, void* workspace,
+                     size_t workspace_bytes, void* stream);
 
 /* Bytes of workspace as_bin_rows_by_degree needs for n rows. */
 size_t as_bin_workspace_bytes(int64_t n);

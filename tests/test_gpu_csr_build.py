@@ -60,6 +60,46 @@ def test_ids_outside_the_rows_end_behind_the_last_row():
     assert col.tolist() == [2, 6, 4, 0, 1, 3, 5] and perm.tolist() == col.tolist()
 
 
+@pytest.mark.parametrize("edges", [1, 700, 300000])
+@pytest.mark.parametrize("bad", [None, 500, -2, 1 << 40, -1])
+def test_ids_outside_the_nodes_are_refused_as_on_the_cpu(edges, bad):
+    nodes = 500
+    ids = torch.from_numpy(np.random.default_rng(edges).integers(0, nodes, size=(2, edges)))
+    ids[:, edges // 2] = nodes - 1
+    for rows_by, end in (("dst", 1), ("src", 0)):
+        host = ids.clone()
+        if bad is not None:
+            host[end, edges * 2 // 3] = bad
+        for build in (edge_index_to_csr, csr_with_edge_order):
+            if bad is None or bad == -1:  # -1 is counted ahead of the first row
+                want = build(host, nodes, rows_by=rows_by)
+                got = build(host.cuda(), nodes, rows_by=rows_by)
+                assert all(torch.equal(g.cpu(), w) for g, w in zip(got, want))
+            else:
+                for where in (host, host.cuda()):
+                    with pytest.raises(IndexError):
+                        build(where, nodes, rows_by=rows_by)
+
+
+@pytest.mark.parametrize("what", ["column n", "column -1", "far column", "edges past the last row", "descending"])
+def test_malformed_graphs_have_no_transpose(what):
+    crow, col = case_graph(3000, 20, seed=4)
+    if "column" in what:
+        col[col.size // 2] = {"column n": 3000, "column -1": -1, "far column": 1 << 33}[what]
+    elif what == "descending":
+        crow[1500] = crow[-1]
+    else:
+        crow[-1] -= 1
+    d = to_dev(crow, col)
+    assert _native.csr_build_supported(*d, 3000)
+    with pytest.raises(RuntimeError, match="malformed CSR"):
+        _autograd._build_transpose(*d)
+    # the next call is not affected
+    crow, col = case_graph(3000, 20, seed=4)
+    host = _autograd._build_transpose(torch.from_numpy(crow), torch.from_numpy(col))
+    assert all(torch.equal(d.cpu(), h) for d, h in zip(_autograd._build_transpose(*to_dev(crow, col)), host))
+
+
 def test_what_keeps_the_torch_composition():
     ids = torch.zeros(4, dtype=torch.long, device="cuda")
     assert _native.csr_build_supported(ids, ids, 3)
