@@ -8,6 +8,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from autosage_amd import _autograd, _native
 from autosage_amd.utils.csr import csr_with_edge_order, edge_index_to_csr
@@ -112,6 +113,9 @@ def test_what_keeps_the_torch_composition():
     empty = torch.zeros((2, 0), dtype=torch.long, device="cuda")
     crow, col = edge_index_to_csr(empty, 3)
     assert crow.tolist() == [0, 0, 0, 0] and col.numel() == 0
+    traced = make_fx(lambda e: edge_index_to_csr(e, 3))(torch.tensor([[0, 1, 2], [2, 2, 0]], device="cuda"))
+    other = torch.tensor([[1, 0, 2], [0, 1, 0]], device="cuda")
+    assert all(torch.equal(t, e) for t, e in zip(traced(other), edge_index_to_csr(other, 3)))
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         captured = _native.csr_build_supported(ids, ids, 3)
