@@ -373,28 +373,34 @@ def spmm_csr_impl(crow, col, val, x):
     return y
 
 
-# fp32 spmm_csr asks for the longest row (once per graph: one host sync,
-# memoised) where it changes the launch by more than the question costs: wide
-# rows of 12 edges or more on graphs of this many edges.
+# fp32 spmm_csr asks for the longest row where it changes the launch by more than
+# the question costs: wide rows of 12 edges or more on graphs of this many edges.
 _EVEN_ROWS_MIN_NNZ = 1 << 19
+_LONGEST_ROW_MEMO = GraphMemo("longest_row", max_entries=64)
 
 
 def _even_rows(crow: torch.Tensor, col: torch.Tensor, f: int) -> bool:
     """Whether the graph is known to have no row of as_spmm_long_row() edges
-    (the same bits either way).  A stream capture takes no sync: only what
-    an earlier call found out counts there."""
+    (the same bits either way).  The first call on a graph asks the device, and
+    a call that finds the answer there uses it; none waits for it.  Nobody asks
+    under stream capture, about row pointers without a version counter
+    (``torch.inference_mode``) or about a copy made for this call, which the
+    next call would not meet again."""
     n = crow.numel() - 1
-    if not 32 < f <= 256 or col.numel() < max(_EVEN_ROWS_MIN_NNZ, 12 * n):
+    # as_spmm_csr_rows_f32 looks at the hint for these widths only
+    if not (32 < f <= 256 and (f <= 64 or f % 2 == 0)) or col.numel() < max(_EVEN_ROWS_MIN_NNZ, 12 * n):
         return False
-
-    def compute() -> int:
-        return int((crow[1:] - crow[:-1]).amax().item())
-
-    if torch.cuda.is_current_stream_capturing():
-        longest = _ROW_COUNT_MEMO.peek((crow,), "longest")
-    else:
-        longest = _ROW_COUNT_MEMO.get((crow,), "longest", compute)
-    return longest is not None and longest < library().as_spmm_long_row()
+    if crow.is_inference() or not _env_vec4():
+        return False
+    longest = _LONGEST_ROW_MEMO.peek((crow,), None)
+    if longest is None:
+        with _on(crow.device):
+            if not getattr(crow, "_autosage_copy", False) and not torch.cuda.is_current_stream_capturing():
+                longest = torch.full((1,), -1, dtype=torch.long, device="cpu", pin_memory=True)
+                longest.copy_((crow[1:] - crow[:-1]).amax(dim=0, keepdim=True), non_blocking=True)
+                _LONGEST_ROW_MEMO.put((crow,), None, longest)
+        return False
+    return 0 <= longest.item() < library().as_spmm_long_row()
 
 
 def spmm_csr_split_impl(crow, col, val, x, feature_tile, warps_per_block, hub_threshold):

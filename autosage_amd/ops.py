@@ -110,6 +110,7 @@ def _normalize_csr(crow, col, val, x):
     # tensors already in shape are passed through as they are (no new tensor)
     if crow.dtype != torch.long or not crow.is_contiguous():
         crow = crow.to(dtype=torch.long).contiguous()
+        crow._autosage_copy = True  # not worth a question about the graph
     if col.dtype != torch.long or not col.is_contiguous():
         col = col.to(dtype=torch.long).contiguous()
     if not x.is_contiguous():

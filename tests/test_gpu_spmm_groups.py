@@ -9,8 +9,9 @@ import numpy as np
 import pytest
 import torch
 
+import autosage_amd
 import oracle
-from autosage_amd import _native
+from autosage_amd import _autograd, _native
 from gpu_common import bitwise_equal, mismatch_report, require_gpu, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -82,7 +83,8 @@ def test_spmm_groups_hand_out_rows(features, mean):
 @pytest.mark.parametrize("long_row", [False, True])
 @pytest.mark.parametrize("features", [40, 47, 96, 128, 200])
 def test_spmm_rows_known_to_be_even(features, long_row):
-    """Above 2^19 edges the op asks for the longest row once per graph."""
+    """Above 2^19 edges the op asks for the longest row once per graph, and knows
+    it from the next call on that finds the answer."""
     rows = 40000
     lengths = np.full(rows, 14)
     if long_row:
@@ -92,10 +94,79 @@ def test_spmm_rows_known_to_be_even(features, long_row):
     x = rng.standard_normal((rows, features)).astype(np.float32)
     val = rng.standard_normal(col.size).astype(np.float32)
     d_crow, d_col, d_val, d_x = to_dev(crow, col, val, x)
-    assert _native._even_rows(d_crow, d_col, features) is not long_row
-    got = torch.ops.autosage.spmm_csr(d_crow, d_col, d_val, d_x)
     ref = oracle.spmm_seq(crow, col, val, x)
-    assert bitwise_equal(got, ref), mismatch_report(got, ref)
+    for known in (False, not long_row, not long_row):
+        torch.cuda.synchronize()
+        assert _native._even_rows(d_crow, d_col, features) is known
+        got = torch.ops.autosage.spmm_csr(d_crow, d_col, d_val, d_x)
+        assert bitwise_equal(got, ref), mismatch_report(got, ref)
+
+
+def _even_graph(features):
+    rows = 40000
+    crow, col, rng = _graph(np.full(rows, 14), features)
+    x = rng.standard_normal((rows, features)).astype(np.float32)
+    return to_dev(crow, col, x), oracle.spmm_seq(crow, col, None, x)
+
+
+def test_no_call_waits_for_the_longest_row():
+    """A new graph, its transpose in the backward and int32 indices, in the range
+    where the longest row matters: nothing waits for the device."""
+    (crow, col, x), ref = _even_graph(64)
+    autosage_amd.spmm_csr(*(t.clone() for t in (crow, col)), None, x)  # loads what the first call loads
+    x.requires_grad_(True)
+    crow_t, col_t, _ = _autograd.csr_transpose(crow, col)
+    mode = torch.cuda.get_sync_debug_mode()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        out = [autosage_amd.spmm_csr(crow, col, None, x)]
+        (grad,) = torch.autograd.grad(out[0], (x,), x.detach())
+        for _ in range(2):
+            out.append(autosage_amd.spmm_csr(crow.int(), col.int(), None, x))
+    finally:
+        torch.cuda.set_sync_debug_mode(mode)
+    assert all(bitwise_equal(o, ref) for o in out)
+    assert torch.equal(grad, torch.ops.autosage.spmm_csr(crow_t, col_t, None, x.detach()))
+
+
+def test_nothing_is_asked_about_copies_and_widths_without_a_choice(monkeypatch):
+    (crow, col, x), _ = _even_graph(64)
+    entries = len(_native._LONGEST_ROW_MEMO)
+    autosage_amd.spmm_csr(crow.int(), col.int(), None, x)
+    assert not _native._even_rows(crow, col, 65) and not _native._even_rows(crow, col, 32)
+    monkeypatch.setenv("AUTOSAGE_VEC4", "0")
+    assert not _native._even_rows(crow, col, 64)
+    assert len(_native._LONGEST_ROW_MEMO) == entries
+
+
+@pytest.mark.parametrize("exact_shard", [False, True])
+def test_graphs_made_in_inference_mode(exact_shard):
+    """Tensors without a version counter."""
+    with torch.inference_mode():
+        (crow, col, x), ref = _even_graph(64)
+        call = ((lambda: _native.spmm_csr_rect_impl(crow, col, None, x, exact=True)) if exact_shard
+                else (lambda: autosage_amd.spmm_csr(crow, col, None, x)))
+        assert crow.is_inference()
+        for _ in range(2):
+            assert bitwise_equal(call(), ref)
+    assert bitwise_equal(call(), ref)
+
+
+def test_the_longest_row_under_capture():
+    (crow, col, x), ref = _even_graph(64)
+    torch.ops.autosage.spmm_csr(crow.clone(), col, None, x)  # loads the kernels
+    y = torch.zeros_like(x)
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for graph in graphs:  # nobody asked; then the answer is there
+        with torch.cuda.graph(graph):
+            y.copy_(torch.ops.autosage.spmm_csr(crow, col, None, x))
+        for _ in range(2):
+            y.zero_()
+            graph.replay()
+            assert bitwise_equal(y, ref)
+        torch.ops.autosage.spmm_csr(crow, col, None, x)
+        torch.cuda.synchronize()
+        assert _native._even_rows(crow, col, 64)
 
 
 @pytest.mark.parametrize("rows", [40, 8191, 8192])
