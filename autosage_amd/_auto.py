@@ -674,55 +674,74 @@ _SHORT_CALL_MS = 0.25
 _BURST = 8
 
 
+def _burst_ms(call) -> float:
+    """The time of one of ``_BURST`` calls back to back."""
+
+    def burst():
+        with torch.no_grad():  # recording a graph would be what is timed
+            for _ in range(_BURST):
+                out = call()
+        return out
+
+    return _time_cuda(burst, warmup=0, iterations=3)["best_ms"] / _BURST
+
+
 def _back_to_back(times: dict[str, float], run_option) -> dict[str, float]:
     """The times of one call each, short ones in a close race timed again as
     calls back to back, as a program runs them: alone, an option of several
     launches waits for each of them on the host (78k rows, 1.4M edges, a row of
     5,000 edges, F = 32: exact in one launch 0.080 ms, column-sliced in four
-    0.086; back to back 0.073 and 0.063)."""
+    0.086; back to back 0.073 and 0.063).  An option that takes more than 1.5
+    times the best one's time alone is out of the race."""
     best = min(times.values())
     close = [key for key in times if times[key] <= 1.5 * best]
     if best >= _SHORT_CALL_MS or len(close) < 2:
         return times
+    return {**times, **{key: _burst_ms(lambda o=json.loads(key): run_option(o)) for key in close}}
 
-    def burst(option):
-        with torch.no_grad():  # recording a graph would be what is timed
-            for _ in range(_BURST):
-                out = run_option(option)
-        return out
 
-    return {**times, **{key: _time_cuda(lambda o=json.loads(key): burst(o), warmup=0, iterations=3)["best_ms"] / _BURST
-                        for key in close}}
+def _race(keys: list[str], run_option, *, warmup: int, iterations: int) -> tuple[dict[str, float], bool]:
+    """(time per option (JSON key), whether calls back to back decided): what
+    every full-graph decision compares, and records."""
+    alone = {
+        key: _time_cuda(lambda o=json.loads(key): run_option(o), warmup=warmup, iterations=iterations)["best_ms"]
+        for key in keys
+    }
+    times = _back_to_back(alone, run_option)
+    return times, times is not alone
 
 
 def _decide_on_full_graph(result: dict[str, Any], options: list[Any], run_option, baseline,
                           inexact: tuple = ()) -> None:
-    """Times each native option on the full graph (1 warmup, best of 3) and
-    the baseline, keeps the fastest native option (a reassociating option of
-    ``inexact`` only when it beats the best bit-exact one by more than
+    """Times each native option on the full graph (1 warmup, best of 3, or back
+    to back) and the baseline, keeps the fastest native option (a reassociating
+    option of ``inexact`` only when it beats the best bit-exact one by more than
     ``_INEXACT_MARGIN``), and falls back to the baseline only when that is
     faster.  `result` gets a ``full_graph`` record; the sampled probe has
     only shortlisted."""
     wall_start = time.perf_counter()
     options = list(dict.fromkeys(json.dumps(o) for o in options))
-    times = {
-        key: _time_cuda(lambda o=json.loads(key): run_option(o), warmup=1, iterations=3)["best_ms"] for key in options
-    }
-    best_key = _prefer_exact(options, _back_to_back(times, run_option), tuple(json.dumps(o) for o in inexact))
+    times, bursts = _race(options, run_option, warmup=1, iterations=3)
+    best_key = _prefer_exact(options, times, tuple(json.dumps(o) for o in inexact))
     best_ms = times[best_key]
     # One baseline call decides when it takes more than twice the best native
-    # time; a closer race gets the full warm timing.  The sampled probe has
-    # already run the baseline, so library set-up is not in this call, and on
-    # large graphs one baseline call costs tens of native ones.
+    # time; a closer race gets the full warm timing, and a short one the timing
+    # of the options.  The sampled probe has already run the baseline, so library
+    # set-up is not in this call, and on large graphs one baseline call costs tens
+    # of native ones.
     baseline_ms = _time_cuda(baseline, warmup=0, iterations=1)["best_ms"]
     baseline_runs = 1
-    if baseline_ms < 2.0 * best_ms:
+    if bursts and baseline_ms < 2.0 * _SHORT_CALL_MS:
+        baseline_ms = _burst_ms(baseline)
+        baseline_runs += 3 * _BURST
+    elif baseline_ms < 2.0 * best_ms:
         baseline_ms = _time_cuda(baseline, warmup=1, iterations=3)["best_ms"]
         baseline_runs = 5
     result["full_graph"] = {
         "autosage_ms": best_ms,
         "baseline_ms": baseline_ms,
         "baseline_runs": baseline_runs,
+        "back_to_back": bursts,
         "candidates": [{"candidate": json.loads(k), "best_ms": times[k]} for k in options],
         "sampled_choice": result.get("candidate"),
         "wall_ms": (time.perf_counter() - wall_start) * 1000.0,
@@ -775,36 +794,25 @@ def calibrate_full(crow, col, val, x, guardrail: float = 0.95) -> tuple[str, dic
     config = SchedulerConfig.from_env(guardrail=guardrail, candidate_count=6)
     baseline, baseline_name = _prepare_spmm_baseline(crow, col, val, x)
     baseline_timing = _time_cuda(baseline, warmup=2, iterations=5)
-    split = native_op("spmm_csr_split") if config.hub_split else None
-    core = native_op("spmm_csr")
-    best, selected = float("inf"), None
-    timings: list[dict[str, Any]] = []
-    if split is not None:
-        for tile, waves, threshold in _spmm_candidates(crow, x.size(1), config):
-            t = _time_cuda(lambda a=tile, b=waves, c=threshold: split(crow, col, val, x, a, b, c), warmup=2, iterations=5)
-            timings.append({"candidate": [tile, waves, threshold], "best_ms": t["best_ms"]})
-            if t["best_ms"] < best:
-                best, selected = t["best_ms"], [tile, waves, threshold]
-    if core is not None:
-        # the whole-graph kernel (candidate None), as in the full-graph decision
-        t = _time_cuda(lambda: core(crow, col, val, x), warmup=2, iterations=5)
-        timings.append({"candidate": None, "best_ms": t["best_ms"]})
-        if t["best_ms"] < best:
-            best, selected = t["best_ms"], None
+    options: list[Any] = []
+    if native_op("spmm_csr_split") is not None and config.hub_split:
+        options += [[int(v) for v in c] for c in _spmm_candidates(crow, x.size(1), config)]
+    # the whole-graph kernel (candidate None), as in the full-graph decision
+    options.append(None)
     if _fslice_eligible(crow, col, x, config):
-        fslice_op = native_op("spmm_csr_fslice")
-        t = _time_cuda(lambda: fslice_op(crow, col, val, x), warmup=2, iterations=5)
-        timings.append({"candidate": FSLICE, "best_ms": t["best_ms"]})
-        if t["best_ms"] < best:
-            best, selected = t["best_ms"], FSLICE
+        options.append(FSLICE)
     if _colslice_eligible(crow, col, x, config):
-        colslice_op = native_op("spmm_csr_colslice")
-        t = _time_cuda(lambda: colslice_op(crow, col, val, x), warmup=2, iterations=5)
-        timings.append({"candidate": COLSLICE, "best_ms": t["best_ms"]})
-        # the reassociating schedule only when it beats every bit-exact one by the margin
-        if t["best_ms"] * (1.0 + _INEXACT_MARGIN) < best:
-            best, selected = t["best_ms"], COLSLICE
-    choice = "autosage" if best <= guardrail * baseline_timing["best_ms"] else "baseline"
+        options.append(COLSLICE)
+    keys = list(dict.fromkeys(json.dumps(o) for o in options))
+    times, bursts = _race(keys, lambda o: _run_spmm_choice("autosage", o, crow, col, val, x), warmup=2, iterations=5)
+    # the reassociating schedule only when it beats every bit-exact one by the margin
+    best_key = _prefer_exact(keys, times, (json.dumps(COLSLICE),))
+    best, selected = times[best_key], json.loads(best_key)
+    timings = [{"candidate": json.loads(key), "best_ms": times[key]} for key in keys]
+    baseline_ms = baseline_timing["best_ms"]
+    if bursts and baseline_ms < 2.0 * _SHORT_CALL_MS:
+        baseline_ms = _burst_ms(baseline)
+    choice = "autosage" if best <= guardrail * baseline_ms else "baseline"
     result = {
         "operation": "spmm",
         "schema_version": AUTOTUNE_SCHEMA_VERSION,
@@ -814,9 +822,9 @@ def calibrate_full(crow, col, val, x, guardrail: float = 0.95) -> tuple[str, dic
         "guardrail": guardrail,
         "configuration": config.tuning_signature(),
         "calibration": "full_graph",
-        "baseline_ms": baseline_timing["best_ms"],
-        "autosage_ms": None if best == float("inf") else best,
-        "speedup": baseline_timing["best_ms"] / best if best not in (0.0, float("inf")) else None,
+        "baseline_ms": baseline_ms,
+        "autosage_ms": best,
+        "speedup": baseline_ms / best if best != 0.0 else None,
         "candidates": timings,
         "from_cache": False,
     }
@@ -1056,9 +1064,10 @@ def _attention_variant(crow, col, q, k, v, scale: float) -> tuple[str, dict[str,
     device = device_signature()
     graph = graph_signature_memo(crow, col, q.size(1), operation, dtype=q.dtype)
     cache = ScheduleCache()
-    times = {}
-    for name, op in (("fused", native_op("csr_attention")), ("colslice", native_op("csr_attention_colslice"))):
-        times[name] = _time_cuda(lambda o=op: o(crow, col, q, k, v, scale), warmup=1, iterations=3)["best_ms"]
+    ops = {"fused": native_op("csr_attention"), "colslice": native_op("csr_attention_colslice")}
+    by_key, _ = _race([json.dumps(name) for name in ops], lambda name: ops[name](crow, col, q, k, v, scale), warmup=1,
+                      iterations=3)
+    times = {name: by_key[json.dumps(name)] for name in ops}
     # the exact stages write and read 12 bytes an edge and keep 4 for the backward:
     # taken where faster by more than two timings of one graph differ
     variant = "fused" if times["fused"] * (1.0 + _STAGES_MARGIN) < times["colslice"] else "colslice"

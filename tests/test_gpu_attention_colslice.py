@@ -15,7 +15,7 @@ import torch
 
 import autosage_amd
 import oracle
-from autosage_amd import _native
+from autosage_amd import _auto, _native
 from tests.gpu_common import case_graph, require_gpu, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -94,7 +94,8 @@ def test_attention_forward_times_and_caches_the_variant(monkeypatch, tmp_path):
     assert info["fused"] and info["variant"] in ("fused", "colslice")
     fg = info["attention"]["full_graph"]
     assert fg["fused_ms"] > 0 and fg["colslice_ms"] > 0
-    assert info["variant"] == min(("fused", "colslice"), key=lambda name: fg[f"{name}_ms"])
+    faster = fg["fused_ms"] * (1.0 + _auto._STAGES_MARGIN) < fg["colslice_ms"]
+    assert info["variant"] == ("fused" if faster else "colslice")
     exact = oracle.attention_f64(crow, col, q, k, v, scale=0.125)
     _check(out.cpu().numpy(), exact)
     again, info2 = autosage_amd.csr_attention_forward(*d, scale=0.125)
