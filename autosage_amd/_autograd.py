@@ -65,7 +65,8 @@ def _build_transpose(crow: torch.Tensor, col: torch.Tensor) -> tuple[torch.Tenso
 # The backward SpMMs run on the feature-sliced kernel where X is beyond the L2s
 # and rows are long (or where it is forced on), else on the whole-graph kernel,
 # which gives long rows workgroups of their own: the same bits (CSR order per
-# output) and no host sync on a new graph's transpose.
+# output), and it waits for nothing on a new graph's transpose.  Fewer than 4
+# features: _narrow_schedule.
 def _spmm(crow, col, val, x, sliced: bool = False):
     if x.dtype != torch.float32:
         # bf16 / fp16: the rounded SpMM, the same bits on any schedule
@@ -78,7 +79,37 @@ def _spmm(crow, col, val, x, sliced: bool = False):
     if _feature_slices_pay(crow, col, x):
         # the same bits, XCD-local on large graphs
         return torch.ops.autosage.spmm_csr_fslice(crow, col, val, x)
+    schedule = _narrow_schedule(crow, col, x)
+    if schedule == "fslice":
+        return torch.ops.autosage.spmm_csr_fslice(crow, col, val, x)
+    if schedule == "split":
+        return torch.ops.autosage.spmm_csr_split(crow, col, val, x, 64 if x.size(1) <= 64 else 128, 2, _NARROW_HUB)
     return torch.ops.autosage.spmm_csr(crow, col, val, x)
+
+
+# The whole-graph kernel gives long rows workgroups of their own from 4 features
+# on; below (and with AUTOSAGE_VEC4=0) it runs them on one wave each, in row order,
+# and on large graphs another schedule is the faster one.  F = 1, us, whole graph /
+# degree split / feature-sliced: 1M rows, 16M edges, longest 10,000 660 / 429 / 453,
+# longest 2,000 471 / 447 / 239, even 378 / 490 / 328; 400k rows, 12M edges, longest
+# 3,000 301 / 251 / 156; 135k rows, 1.9M edges, longest 3,000 120 / 112 / 145.
+_NARROW_ROWS = 1 << 18
+_NARROW_HUB = 2048
+_NARROW_CHAIN = 8192
+
+
+def _narrow_schedule(crow, col, x) -> str:
+    """"fslice", "split" or "rows" for a backward product (the same bits)."""
+    from ._native import _env_vec4, row_counts
+    from .config import SchedulerConfig
+
+    if (x.size(1) >= 4 and _env_vec4()) or crow.numel() <= _NARROW_ROWS:
+        return "rows"
+    if row_counts(crow, _NARROW_HUB, 0)[0] == 0:
+        return "rows"
+    if row_counts(crow, _NARROW_CHAIN, 0)[0] == 0 and SchedulerConfig.from_env().feature_slices != "off":
+        return "fslice"
+    return "split"
 
 
 def _feature_slices_pay(crow, col, x) -> bool:

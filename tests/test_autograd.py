@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import oracle
+from autosage_amd import _autograd
 from autosage_amd._autograd import csr_transpose
 from tests.gpu_common import bitwise_equal, case_graph, require_gpu, to_dev
 
@@ -27,6 +28,41 @@ def test_csr_transpose_matches_dense_transpose():
     assert np.array_equal(perm.numpy(), order)
     assert np.array_equal(t_col.numpy(), rows[order])
     assert np.array_equal(t_crow.numpy(), np.concatenate([[0], np.cumsum(np.bincount(col, minlength=n))]))
+
+
+@pytest.mark.parametrize("rows, longest, features, vec4, schedule", [
+    (1 << 18, 2048, 3, None, "fslice"), (1 << 18, 8191, 1, None, "fslice"), (1 << 18, 8192, 1, None, "split"),
+    (1 << 18, 2047, 1, None, "rows"), ((1 << 18) - 1, 8192, 1, None, "rows"),
+    (1 << 18, 8192, 4, None, "rows"), (1 << 18, 8192, 4, "0", "split"),
+])
+def test_schedule_of_narrow_backward_products(monkeypatch, rows, longest, features, vec4, schedule):
+    if vec4 is not None:
+        monkeypatch.setenv("AUTOSAGE_VEC4", vec4)
+    lengths = torch.ones(rows, dtype=torch.long)
+    lengths[rows // 2] = longest
+    crow = torch.cat([lengths.new_zeros(1), lengths.cumsum(0)])
+    assert _autograd._narrow_schedule(crow, lengths.new_zeros(int(crow[-1])), torch.zeros(rows, features)) == schedule
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("longest", [2500, 9000])
+@pytest.mark.parametrize("features", [1, 3])
+def test_narrow_gradients_on_large_graphs_with_long_rows(features, longest):
+    require_gpu()
+    rows = 1 << 18
+    rng = np.random.default_rng(longest)
+    col = rng.integers(0, rows, size=3 * rows)
+    col[rng.permutation(col.size)[:longest]] = 77  # a hub of the transposed graph
+    crow = np.arange(0, 3 * rows + 1, 3)
+    x, g = (rng.standard_normal((rows, features)).astype(np.float32) for _ in range(2))
+    val = rng.standard_normal(col.size).astype(np.float32)
+    d_crow, d_col, d_val, d_x, d_g = to_dev(crow, col, val, x, g)
+    crow_t, col_t, perm = csr_transpose(d_crow, d_col)
+    assert _autograd._narrow_schedule(crow_t, col_t, d_g) == ("fslice" if longest < 8192 else "split")
+    out = torch.ops.autosage.spmm_csr(d_crow, d_col, d_val, d_x.requires_grad_(True))
+    (grad,) = torch.autograd.grad(out, (d_x,), d_g)
+    want = oracle.spmm_seq(crow_t.cpu().numpy(), col_t.cpu().numpy(), val[perm.cpu().numpy()], g)
+    assert bitwise_equal(grad, want)
 
 
 def test_csr_transpose_memo_is_per_tensor_object():
