@@ -38,17 +38,21 @@ def test_softmax_rows_of_every_length(order):
     got = torch.ops.autosage.csr_row_softmax(d_crow, d_scores)
     ref = oracle.row_softmax(crow, scores)
     assert np.all(np.abs(got.cpu().numpy() - ref) <= 1e-6 + 1e-5 * np.abs(ref))
-    # the denominator's order: an attention over one-hot values computes the
-    # same probabilities in one wave (or four) per row
-    n = lengths.size
-    q = rng.standard_normal((n, 32)).astype(np.float32)
-    k = rng.standard_normal((n, 32)).astype(np.float32)
-    v = rng.standard_normal((n, 8)).astype(np.float32)
-    col = rng.integers(0, n, size=int(crow[-1])).astype(np.int64)
-    d_col, d_q, d_k, d_v = to_dev(col, q, k, v)
-    probs = torch.ops.autosage.csr_row_softmax(d_crow, torch.ops.autosage.sddmm_csr(d_crow, d_col, d_q, d_k))
-    fused = torch.ops.autosage.csr_attention(d_crow, d_col, d_q, d_k, d_v, 1.0)
-    assert torch.equal(torch.ops.autosage.spmm_csr(d_crow, d_col, probs, d_v), fused)
+    # bit for bit: 64 chains of every 64th exponential, a 32/16/8/4/2/1 butterfly,
+    # an IEEE division (the exponential itself is the device's)
+    maxima = np.array([scores[b:e].max(initial=-np.inf) for b, e in zip(crow, crow[1:])], dtype=np.float32)
+    exps = torch.exp(torch.from_numpy(scores - np.repeat(maxima, lengths)).cuda()).cpu().numpy()
+    want = np.empty_like(scores)
+    for row, (b, e) in enumerate(zip(crow, crow[1:])):
+        chains = np.zeros((-(-(e - b) // 64), 64), dtype=np.float32)
+        chains.reshape(-1)[: e - b] = exps[b:e]
+        d = np.zeros(64, dtype=np.float32)
+        for step in chains:
+            d = d + step
+        for o in (32, 16, 8, 4, 2, 1):
+            d = d + d[np.arange(64) ^ o]
+        want[b:e] = exps[b:e] / d[0] if e > b else 0
+    assert bitwise_equal(got, want)
     grad = rng.standard_normal(scores.size).astype(np.float32)
     (d_grad,) = to_dev(grad)
     back = csr_row_softmax_backward_impl(d_crow, got, d_grad)
