@@ -907,8 +907,9 @@ def sddmm_csr_auto(
     core = native_op("sddmm_csr")
     split_calls = []
     if split is not None:
-        pairs = dict.fromkeys((w, h) for _, w, h in _spmm_candidates(s_crow, query.size(1), config))
-        for waves, threshold in pairs:
+        # one pair: fp32 SDDMM runs the same blocks of edges for every pair, and
+        # the baseline is what it races
+        for _, waves, threshold in _spmm_candidates(s_crow, query.size(1), config)[:1]:
             split_calls.append(([waves, threshold], lambda w=waves, h=threshold: split(s_crow, s_col, s_q, s_k, w, h)))
     core_call = (lambda: core(s_crow, s_col, s_q, s_k)) if (split is None and core is not None) else None
     probe = _probe_and_choose(
@@ -922,17 +923,12 @@ def sddmm_csr_auto(
     )
     result = _result_dict("sddmm", config, probe, baseline_name, s_crow, s_col, sample_ms)
     if config.full_graph_check and split is not None:
-        # the sampled best pair and the pair of the full graph's preferred
-        # candidate, on the full graph
-        # (fp32 SDDMM runs the same blocks of edges for every pair: their
-        # times differ by noise only, and the baseline is what they are
-        # compared with)
+        # the pair of the full graph's preferred candidate
         _, waves, threshold = _full_graph_candidate(crow, query.size(1), config)
         if config.hub_threshold is None:
             threshold = max(threshold, _SDDMM_MIN_HUB_DEGREE)
-        options = ([probe["chosen"]] if probe["chosen"] is not None else []) + [[waves, threshold]]
         full_baseline, _ = _prepare_sddmm_baseline(crow, col, query, key)
-        _decide_on_full_graph(result, options, lambda o: _run_sddmm_choice("autosage", o, crow, col, query, key),
+        _decide_on_full_graph(result, [[waves, threshold]], lambda o: _run_sddmm_choice("autosage", o, crow, col, query, key),
                               full_baseline)
     output = _run_sddmm_choice(result["choice"], result["candidate"], crow, col, query, key)
     if config.cache:

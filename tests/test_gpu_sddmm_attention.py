@@ -222,6 +222,18 @@ def test_schedulers_decide_on_the_full_graph(monkeypatch, tmp_path):
     assert "full_graph" not in info0
 
 
+def test_fp32_sddmm_races_the_baseline_alone(monkeypatch, tmp_path):
+    """Its schedules are one kernel, so one of them is timed."""
+    monkeypatch.setenv("AUTOSAGE_CACHE_DIR", str(tmp_path))
+    crow, col = case_graph(30000, 24, seed=17, hubs=8, hub_degree=8000)
+    q, kk = _qk(30000, 64, seed=5)
+    d_crow, d_col, d_q, d_k = to_dev(crow, col, q, kk)
+    scores, info = sddmm_csr_auto(d_crow, d_col, d_q, d_k)
+    assert len(info["candidates"]) == 1 and len(info["full_graph"]["candidates"]) == 1
+    again, replay = sddmm_csr_auto(d_crow, d_col, d_q, d_k)
+    assert replay["from_cache"] and replay["candidate"] == info["candidate"] and torch.equal(scores, again)
+
+
 def test_calibrate_full_times_every_option_and_is_replayed(monkeypatch, tmp_path):
     monkeypatch.setenv("AUTOSAGE_CACHE_DIR", str(tmp_path))
     crow, col = case_graph(30000, 24, seed=17, hubs=8, hub_degree=8000)
