@@ -215,6 +215,7 @@ def _spmm_candidates(crow: torch.Tensor, feature_width: int, config: SchedulerCo
 
 COLSLICE = "colslice"  # candidate value of the column-sliced SpMM
 FSLICE = "fslice"  # candidate value of the feature-sliced SpMM (bit-exact)
+SDDMM_ROWS = "rows"  # candidate value of the SDDMM by rows (bit-exact)
 # The column-sliced SpMM reassociates each row's sum (fp64 partials, one
 # rounding); the other native schedules keep the reference's CSR-order fp32
 # chain.  The full-graph decision takes the column-sliced one only when it
@@ -306,8 +307,8 @@ def _cached_native_available(operation: str, choice: str, candidate) -> bool:
         return native_op(operation) is not None
     if candidate == COLSLICE:
         return native_op(operation + "_colslice") is not None
-    if candidate == FSLICE:
-        return native_op(operation + "_fslice") is not None
+    if candidate in (FSLICE, SDDMM_ROWS):
+        return native_op(f"{operation}_{candidate}") is not None
     return native_op(operation + ("_split" if candidate is not None else "")) is not None
 
 
@@ -395,7 +396,9 @@ def _run_spmm_choice(choice, candidate, crow, col, val, x) -> torch.Tensor:
 def _run_sddmm_choice(choice, candidate, crow, col, query, key) -> torch.Tensor:
     if choice == "autosage":
         out = None
-        if candidate is not None:
+        if candidate == SDDMM_ROWS:
+            out = _op_call("sddmm_csr_rows", (crow, col, query, key), (query, key))
+        elif candidate is not None:
             out = _op_call("sddmm_csr_split", (crow, col, query, key, *map(int, candidate)), (query, key))
         if out is None:
             out = _op_call("sddmm_csr", (crow, col, query, key), (query, key))
@@ -857,6 +860,23 @@ def _normalize_sddmm(crow, col, query, key):
     return crow, col, query, key
 
 
+# The product by rows beats the blocks of edges by 2-6 % on keys beyond the caches
+# with rows of 40 edges or more and columns without a pattern, which sizes do not
+# tell (figures at the kernel): timed from these sizes on (300k rows of 100 edges, F =
+# 64, a key of 77 MB 1102 against 1081 us; 100k rows of 50, F = 128, 51 MB 354 / 356;
+# 1M rows of 16, F = 128 1289 / 1299; F = 32 985 / 1052).
+_SDDMM_ROWS_MIN_KEY_BYTES = 64 << 20
+_SDDMM_ROWS_MIN_MEAN_DEGREE = 32
+
+
+def _sddmm_rows_eligible(crow, col, query, key) -> bool:
+    from ._native import sddmm_rows_supported
+
+    n, f = query.shape
+    return (native_op("sddmm_csr_rows") is not None and sddmm_rows_supported(query, key) and f >= 64
+            and n * f * 4 >= _SDDMM_ROWS_MIN_KEY_BYTES and col.numel() >= _SDDMM_ROWS_MIN_MEAN_DEGREE * n)
+
+
 def sddmm_csr_auto(
     crow: torch.Tensor,
     col: torch.Tensor,
@@ -907,8 +927,8 @@ def sddmm_csr_auto(
     core = native_op("sddmm_csr")
     split_calls = []
     if split is not None:
-        # one pair: fp32 SDDMM runs the same blocks of edges for every pair, and
-        # the baseline is what it races
+        # one pair: the split runs the same blocks of edges for every pair, and
+        # the baseline is what it races on the sample
         for _, waves, threshold in _spmm_candidates(s_crow, query.size(1), config)[:1]:
             split_calls.append(([waves, threshold], lambda w=waves, h=threshold: split(s_crow, s_col, s_q, s_k, w, h)))
     core_call = (lambda: core(s_crow, s_col, s_q, s_k)) if (split is None and core is not None) else None
@@ -923,12 +943,14 @@ def sddmm_csr_auto(
     )
     result = _result_dict("sddmm", config, probe, baseline_name, s_crow, s_col, sample_ms)
     if config.full_graph_check and split is not None:
-        # the pair of the full graph's preferred candidate
+        # the pair of the full graph's preferred candidate and, where it may be
+        # the faster one, the product by rows
         _, waves, threshold = _full_graph_candidate(crow, query.size(1), config)
         if config.hub_threshold is None:
             threshold = max(threshold, _SDDMM_MIN_HUB_DEGREE)
         full_baseline, _ = _prepare_sddmm_baseline(crow, col, query, key)
-        _decide_on_full_graph(result, [[waves, threshold]], lambda o: _run_sddmm_choice("autosage", o, crow, col, query, key),
+        options = [[waves, threshold]] + ([SDDMM_ROWS] if _sddmm_rows_eligible(crow, col, query, key) else [])
+        _decide_on_full_graph(result, options, lambda o: _run_sddmm_choice("autosage", o, crow, col, query, key),
                               full_baseline)
     output = _run_sddmm_choice(result["choice"], result["candidate"], crow, col, query, key)
     if config.cache:

@@ -287,7 +287,7 @@ def register() -> None:
     for name in ("spmm_csr", "spmm_csr_split", "spmm_csr_fslice"):
         torch.library.register_autograd(f"autosage::{name}", _spmm_backward, setup_context=_spmm_setup)
     torch.library.register_autograd("autosage::spmm_csr_colslice", _spmm_backward, setup_context=_spmm_sliced_setup)
-    for name in ("sddmm_csr", "sddmm_csr_split"):
+    for name in ("sddmm_csr", "sddmm_csr_split", "sddmm_csr_rows"):
         torch.library.register_autograd(f"autosage::{name}", _sddmm_backward, setup_context=_sddmm_setup)
     torch.library.register_autograd("autosage::csr_row_softmax", _softmax_backward, setup_context=_softmax_setup)
     torch.library.register_autograd("autosage::csr_attention", _attention_backward, setup_context=_attention_setup)

@@ -88,6 +88,8 @@ _SIGNATURES = {
     ),
     "as_sddmm_csr_edges_f32": (
         _c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr]),
+    "as_sddmm_csr_rows_f32": (
+        _c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_size, _c_ptr]),
     "as_sddmm_csr_f32": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr]),
     "as_sddmm_split_workspace_bytes": (_c_size, [_c_i64]),
     "as_sddmm_csr_split_f32": (
@@ -783,6 +785,34 @@ def sddmm_csr_impl(crow, col, query, key):
     return out
 
 
+def sddmm_rows_supported(query, key) -> bool:
+    """Whether ``sddmm_csr_rows`` has a kernel of its own for these (fp32)."""
+    f = query.size(1)
+    return (query.dtype == torch.float32 and 32 <= f <= 256 and f % 32 == 0
+            and query.data_ptr() % 16 == 0 and key.data_ptr() % 16 == 0)
+
+
+def sddmm_csr_rows_impl(crow, col, query, key):
+    """``sddmm_csr`` one wave per row, the same bits; what that kernel does not
+    take runs as ``sddmm_csr``."""
+    check_sddmm_inputs(crow, col, query, key, allow_16=True)
+    n, f = query.shape
+    nnz = col.numel()
+    if n == 0 or nnz == 0 or not sddmm_rows_supported(query, key):
+        return sddmm_csr_impl(crow, col, query, key)
+    _maybe_validate(crow, col)
+    out = torch.empty(nnz, dtype=query.dtype, device=query.device)
+    lib = library()
+    ws = _workspace(lib.as_sddmm_split_workspace_bytes(n), query.device)
+    with _on(query.device):
+        status = lib.as_sddmm_csr_rows_f32(
+            _ptr(crow), _ptr(col), _ptr(query), _ptr(key), _ptr(out), n, nnz, f, _ptr(ws), ws.numel(),
+            _stream(query.device),
+        )
+    _raise(status, "autosage::sddmm_csr_rows")
+    return out
+
+
 def sddmm_csr_split_impl(crow, col, query, key, warps_per_block, hub_threshold):
     check_sddmm_inputs(crow, col, query, key, allow_16=True)
     if query.dtype in DTYPES_16:
@@ -1457,6 +1487,9 @@ _SCHEMAS = {
         "int hub_threshold) -> Tensor",
         sddmm_csr_split_impl,
     ),
+    # sddmm_csr on its other fp32 kernel, which the scheduler may choose
+    "sddmm_csr_rows": (
+        "sddmm_csr_rows(Tensor crow, Tensor col, Tensor query, Tensor key) -> Tensor", sddmm_csr_rows_impl),
     "csr_row_softmax": ("csr_row_softmax(Tensor crow, Tensor scores) -> Tensor", csr_row_softmax_impl),
     "csr_attention": (
         "csr_attention(Tensor crow, Tensor col, Tensor query, Tensor key, Tensor value, float scale=1.0) -> Tensor",

@@ -21,9 +21,9 @@ namespace {
 
 constexpr int kChunkEdges = 2048;  // edges per hub work item
 
-// Work items of the 16-bit split schedule: hub h (order[h],
-// h < counts[0]) is cut into ceil(deg / kChunkEdges) chunks; chunk_off[h] is the exclusive prefix and
-// counts[2] the total.  One workgroup of 1024 threads.
+// Work items of the 16-bit split schedule and of the fp32 product by rows: hub h
+// (order[h], h < counts[0]) is cut into ceil(deg / kChunkEdges) chunks; chunk_off[h]
+// is the exclusive prefix and counts[2] the total.  One workgroup of 1024 threads.
 __global__ __launch_bounds__(1024) void hub_chunk_scan_kernel(const int64_t* __restrict__ crow,
                                                               const int32_t* __restrict__ order,
                                                               int32_t* __restrict__ counts,
@@ -364,6 +364,139 @@ void launch_sddmm_edges(const SddmmArgs& a, int64_t nnz, int64_t n_keys, float s
 // threshold 256), and a pool much smaller than the chunk count leaves the
 // hub pass as a tail behind the light rows.
 constexpr int64_t kHubBlocksMax = 65536;
+
+// ---- fp32 SDDMM by rows --------------------------------------------------------
+// One wave per row, rows of at least kRowsHub edges in chunks of kChunkEdges over
+// workgroups of their own (the first of the launch); the reference's order again.
+// A lane holds its part of the query row (4 features of every 32) and 2 or 4 edges
+// of a lane group are in flight with whole rows of the key.
+//
+// What bounds it: where the key is beyond the caches, the rate of its rows, read
+// whole by one instruction sequence: a few percent ahead of the blocks of edges,
+// which read a row's 128-byte lines one 32-feature block after the other.  us,
+// blocks / rows: 500k rows of 40 edges F = 64 771 / 739, F = 128 1534 / 1481, F =
+// 256 3012 / 2819; 1M rows of 50 F = 64 1949 / 1844; 300k rows of 100 F = 256 4503 /
+// 4232.  Where hubs' columns are cached it falls far behind (1M rows, 50M edges
+// with hubs in the columns too, F = 64 819 / 1494), and with short rows as well (1M
+// rows of 6, F = 64 274 / 542), so the scheduler times it on graphs that may suit it
+// and nothing runs it unasked.
+constexpr int64_t kRowsHub = 1024;
+constexpr int kRowsLanes = 8;  // per edge: lane j holds partials 4j .. 4j + 3
+
+__device__ __forceinline__ float row_dot_tree(float (&p)[4]) {
+#pragma unroll
+  for (int o = 4; o >= 1; o >>= 1) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) p[s] += __shfl_xor(p[s], o, kWave);
+  }
+  return (p[0] + p[2]) + (p[1] + p[3]);
+}
+
+// The dot products of edges first + 8u + lane group (u < UE) below end.
+template <int MF, int UE>
+__device__ __forceinline__ void row_dots(const int64_t* __restrict__ col, const float* __restrict__ key,
+                                         float* __restrict__ out, int64_t F, const FVec<4> (&qv)[MF], int64_t first,
+                                         int64_t end, int g, int j) {
+  constexpr int NG = kWave / kRowsLanes;
+  FVec<4> kv[UE][MF];
+#pragma unroll
+  for (int u = 0; u < UE; ++u) {
+    const int64_t e = first + u * NG + g;
+    const int c = static_cast<int>(col[e < end ? e : end - 1]);
+    const float* kr = key + row_offset(c, F) + 4 * j;
+#pragma unroll
+    for (int m = 0; m < MF; ++m) kv[u][m] = load_vec<4>(kr + 32 * m);
+  }
+#pragma unroll
+  for (int u = 0; u < UE; ++u) {
+    float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) p[s] = __builtin_fmaf(qv[m].v[s], kv[u][m].v[s], p[s]);
+    }
+    const float d = row_dot_tree(p);
+    const int64_t e = first + u * NG + g;
+    if (e < end && j == 0) out[e] = d;
+  }
+}
+
+template <int MF>
+__global__ __launch_bounds__(kBlock) void sddmm_rows_kernel(
+    const int64_t* __restrict__ crow, const int64_t* __restrict__ col, const float* __restrict__ query,
+    const float* __restrict__ key, float* __restrict__ out, int64_t n, int64_t F, const int32_t* __restrict__ order,
+    const int32_t* __restrict__ counts, const int32_t* __restrict__ chunk_off, int64_t hub_blocks,
+    int64_t block_base) {
+  constexpr int NG = kWave / kRowsLanes;
+  const int lane = lane_id();
+  const int g = lane / kRowsLanes;
+  const int j = lane % kRowsLanes;
+  const int wave = wave_in_block();
+  const int64_t block = block_base + blockIdx.x;
+  FVec<4> qv[MF];
+  auto load_query = [&](int64_t row) {
+#pragma unroll
+    for (int m = 0; m < MF; ++m) qv[m] = load_vec<4>(query + row * F + 32 * m + 4 * j);
+  };
+  if (block < hub_blocks) {
+    const int64_t hubs = counts[0];
+    const int64_t items = counts[2];
+    for (int64_t item = block; item < items; item += hub_blocks) {
+      int64_t lo = 0;
+      int64_t hi = hubs - 1;
+      while (lo < hi) {
+        const int64_t mid = (lo + hi + 1) >> 1;
+        if (chunk_off[mid] <= item) lo = mid;
+        else hi = mid - 1;
+      }
+      const int64_t row = uniform_i64(order[lo]);
+      const int64_t cs = uniform_i64(crow[row]) + (item - uniform_i64(chunk_off[lo])) * kChunkEdges;
+      const int64_t re = uniform_i64(crow[row + 1]);
+      const int64_t ce = cs + kChunkEdges < re ? cs + kChunkEdges : re;
+      load_query(row);
+      for (int64_t b = cs + wave * NG; b < ce; b += kWavesPerBlock * NG)
+        row_dots<MF, 1>(col, key, out, F, qv, b, ce, g, j);
+    }
+    return;
+  }
+  const int64_t row = (block - hub_blocks) * kWavesPerBlock + wave;
+  if (row >= n) return;
+  const int64_t rs = uniform_i64(crow[row]);
+  const int64_t re = uniform_i64(crow[row + 1]);
+  if (re - rs >= kRowsHub || re <= rs) return;
+  constexpr int UE = MF <= 2 ? 4 : 2;
+  load_query(row);
+  for (int64_t b = rs; b < re; b += NG * UE) row_dots<MF, UE>(col, key, out, F, qv, b, re, g, j);
+}
+
+bool sddmm_rows_fit(const SddmmArgs& a) {
+  return a.f % 32 == 0 && a.f >= 32 && a.f <= 256 && aligned(a.q, 16) && aligned(a.k, 16);
+}
+
+// hub_blocks workgroups for the chunks of hub rows (an upper bound of them; 0: no
+// row can have kRowsHub edges, order, counts and chunk_off are not read).
+void launch_sddmm_rows(const SddmmArgs& a, int64_t hub_blocks, const int32_t* order, const int32_t* counts,
+                       const int32_t* chunk_off, hipStream_t s) {
+  const int64_t blocks = hub_blocks + (a.n + kWavesPerBlock - 1) / kWavesPerBlock;
+  for (int64_t b0 = 0; b0 < blocks; b0 += kMaxBlocksPerLaunch) {
+    const int64_t nb = blocks - b0 < kMaxBlocksPerLaunch ? blocks - b0 : kMaxBlocksPerLaunch;
+    const dim3 grid(static_cast<unsigned>(nb));
+#define AS_ROWS(MF)                                                                                              \
+  hipLaunchKernelGGL(sddmm_rows_kernel<MF>, grid, dim3(kBlock), 0, s, a.crow, a.col, a.q, a.k, a.out, a.n, a.f, order, \
+                     counts, chunk_off, hub_blocks, b0)
+    switch (static_cast<int>(a.f / 32)) {
+      case 1: AS_ROWS(1); break;
+      case 2: AS_ROWS(2); break;
+      case 3: AS_ROWS(3); break;
+      case 4: AS_ROWS(4); break;
+      case 5: AS_ROWS(5); break;
+      case 6: AS_ROWS(6); break;
+      case 7: AS_ROWS(7); break;
+      default: AS_ROWS(8); break;
+    }
+#undef AS_ROWS
+  }
+}
 
 // ---- bf16 / fp16 SDDMM -------------------------------------------------------
 // out[e] = the fp64 sum of the exact products q[row(e), f]·k[col(e), f],
@@ -982,6 +1115,38 @@ int as_sddmm_csr_edges_f32(const int64_t* crow, const int64_t* col, const float*
   if (f == 0) return as::fail(AS_ERR_UNSUPPORTED, "SDDMM with zero features is handled by the caller");
   as::launch_sddmm_edges(a, nnz, n_keys, 1.f, static_cast<hipStream_t>(stream));
   return as::check_launch("sddmm_csr");
+}
+
+int as_sddmm_csr_rows_f32(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,
+                          int64_t n, int64_t nnz, int64_t f, void* workspace, size_t workspace_bytes, void* stream) {
+  as::clear_error();
+  as::SddmmArgs a{crow, col, query, key, out, n, f};
+  int st = as::validate_sddmm(a, nnz);
+  if (st != AS_OK) return st;
+  if (n == 0 || nnz == 0) return AS_OK;
+  if (!as::sddmm_rows_fit(a))
+    return as::fail(AS_ERR_UNSUPPORTED, "SDDMM by rows takes multiples of 32 features up to 256, 16-byte aligned");
+  if (workspace == nullptr || workspace_bytes < as::sddmm_split_ws(n))
+    return as::fail(AS_ERR_WORKSPACE, "SDDMM by rows needs %zu workspace bytes, got %zu", as::sddmm_split_ws(n),
+                    workspace_bytes);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  int32_t* order = reinterpret_cast<int32_t*>(ws);
+  const size_t order_bytes = as::align_up(static_cast<size_t>(n) * sizeof(int32_t), 256);
+  int32_t* counts = reinterpret_cast<int32_t*>(ws + order_bytes);
+  int32_t* chunk_off = reinterpret_cast<int32_t*>(ws + as::spmm_split_workspace_bytes(n));
+  int64_t hubs = nnz / as::kRowsHub;
+  if (hubs > n) hubs = n;
+  int64_t hub_blocks = 0;
+  if (hubs > 0) {
+    st = as::launch_bin_rows(crow, n, as::kRowsHub, 1, 1, order, counts, ws + order_bytes + 256, s);
+    if (st != AS_OK) return st;
+    hipLaunchKernelGGL(as::hub_chunk_scan_kernel, dim3(1), dim3(1024), 0, s, crow, order, counts, chunk_off);
+    hub_blocks = nnz / as::kChunkEdges + hubs;
+    if (hub_blocks > as::kHubBlocksMax) hub_blocks = as::kHubBlocksMax;
+  }
+  as::launch_sddmm_rows(a, hub_blocks, order, counts, chunk_off, s);
+  return as::check_launch("sddmm_csr_rows");
 }
 
 int as_sddmm_csr_f32(const int64_t* crow, const int64_t* col, const float* query, const float* key, float* out,

@@ -1249,6 +1249,8 @@ def bench_other(args, device) -> dict:
                 lambda a=waves, b=thr: torch.ops.autosage.sddmm_csr_split(crow, col, q, k, a, b))
         whole = "whole" if dt == torch.float32 else "edges"
         variants[whole] = lambda: torch.ops.autosage.sddmm_csr(crow, col, q, k)
+        if dt == torch.float32:
+            variants["rows"] = lambda: torch.ops.autosage.sddmm_csr_rows(crow, col, q, k)
         calib = {}
         chosen = calibrate(variants, calib) if args.variant in ("calibrated", "auto") else args.variant
         step = variants[chosen]
@@ -1262,7 +1264,7 @@ def bench_other(args, device) -> dict:
             _, info = sddmm_csr_auto(crow, col, q, k)
             cand = info.get("candidate")
             chosen = "baseline" if info.get("choice") != "autosage" else (
-                whole if cand is None else ",".join(map(str, cand)))
+                whole if cand is None else cand if isinstance(cand, str) else ",".join(map(str, cand)))
             step = lambda: sddmm_csr_auto(crow, col, q, k)[0]  # noqa: E731
         ms, samples = time_steps(step, args.steps, args.warmup)
         flops = 2.0 * w.nnz * f

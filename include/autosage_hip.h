@@ -496,8 +496,19 @@ int as_sddmm_csr_edges_f32(const int64_t* crow, const int64_t* col,
                            int64_t n, int64_t n_keys, int64_t nnz, int64_t f,
                            void* stream);
 
-/* Bytes of workspace as_sddmm_csr_split_f32 needs for n rows. */
+/* Bytes of workspace as_sddmm_csr_split_f32 and as_sddmm_csr_rows_f32 need for
+ * n rows. */
 size_t as_sddmm_split_workspace_bytes(int64_t n);
+
+/* as_sddmm_csr_f32 (the same bits) one wave per row, rows of 1024 edges or
+ * more in chunks over workgroups: a few percent ahead of the blocks of edges
+ * on long rows whose columns name a key beyond the caches without a pattern,
+ * and behind elsewhere.  f a multiple of 32 up to 256, query and key 16-byte
+ * aligned (else AS_ERR_UNSUPPORTED). */
+int as_sddmm_csr_rows_f32(const int64_t* crow, const int64_t* col,
+                          const float* query, const float* key, float* out,
+                          int64_t n, int64_t nnz, int64_t f, void* workspace,
+                          size_t workspace_bytes, void* stream);
 
 /* Degree-split SDDMM.  Replaces sddmm_csr_split
  * (csrc/sddmm_csr_op.cu:136-187), op schema :193-195.  The settings and the
