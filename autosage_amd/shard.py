@@ -84,7 +84,9 @@ def spmm_csr_shard(crow: torch.Tensor, col: torch.Tensor, val: Optional[torch.Te
         raise ValueError("x must have shape [N, F]")
     if crow.dtype not in (torch.int32, torch.int64) or col.dtype not in (torch.int32, torch.int64):
         raise TypeError("crow and col must use integer indices")
-    crow = crow.to(torch.long).contiguous()
+    if crow.dtype != torch.long or not crow.is_contiguous():
+        crow = crow.to(torch.long).contiguous()
+        crow._autosage_copy = True  # not worth a question about the shard
     col = col.to(torch.long).contiguous()
     if val is not None:
         val = val.to(x.dtype).contiguous()

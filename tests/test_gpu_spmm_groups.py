@@ -11,7 +11,7 @@ import torch
 
 import autosage_amd
 import oracle
-from autosage_amd import _autograd, _native
+from autosage_amd import _autograd, _native, shard
 from gpu_common import bitwise_equal, mismatch_report, require_gpu, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -133,6 +133,7 @@ def test_nothing_is_asked_about_copies_and_widths_without_a_choice(monkeypatch):
     (crow, col, x), _ = _even_graph(64)
     entries = len(_native._LONGEST_ROW_MEMO)
     autosage_amd.spmm_csr(crow.int(), col.int(), None, x)
+    shard.spmm_csr_shard(crow.int(), col.int(), None, x, exact=True)
     assert not _native._even_rows(crow, col, 65) and not _native._even_rows(crow, col, 32)
     monkeypatch.setenv("AUTOSAGE_VEC4", "0")
     assert not _native._even_rows(crow, col, 64)
