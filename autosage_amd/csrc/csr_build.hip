@@ -16,8 +16,9 @@
 // sort is already queued behind it, and not for the sort.
 //
 // What bounds it: the sort's passes (8 bits each).  us, torch composition (with its
-// host syncs) -> here: 40k nodes, 400k edges CSR 204 -> 50, transpose 322 -> 56; 1M nodes,
-// 16M edges 2514 -> 812 and 2766 -> 873; 114M edges 17.0 -> 5.3 and 17.7 -> 5.6 ms.
+// host syncs) -> here: 40k nodes, 400k edges CSR 204 -> 60, transpose 322 -> 64 (without
+// the check 53 and 59); without it 1M nodes, 16M edges 2514 -> 812 and 2766 -> 873; 114M
+// edges 17.0 -> 5.3 and 17.7 -> 5.6 ms.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
 #include <rocprim/iterator/transform_iterator.hpp>
