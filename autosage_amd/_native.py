@@ -1382,13 +1382,14 @@ def csr_build_supported(rows: torch.Tensor, cols: torch.Tensor, n: int) -> bool:
     contiguous int64 CUDA vectors of the sizes the native sort covers, outside
     tracing, functorch transforms, dispatch modes and stream capture (the sort
     may record memsets), which keep the torch composition."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False  # before what a tracer would follow
     if not (type(rows) is torch.Tensor and type(cols) is torch.Tensor and rows.is_cuda and cols.is_cuda
             and rows.get_device() == cols.get_device()
             and rows.dtype is torch.long and cols.dtype is torch.long and rows.dim() == 1 and cols.dim() == 1
             and rows.is_contiguous() and cols.is_contiguous()
             and 0 < n and 0 < cols.numel() and n + cols.numel() < 2**31 - 4097
             and _LIB is not None and _is_wrapped is not None and not _is_wrapped(rows) and not _is_wrapped(cols)
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and torch._C._len_torch_dispatch_stack() == 0):
         return False
     with _on(rows.device):

@@ -28,7 +28,7 @@ def _row_and_column_ids(edge_index: torch.Tensor, rows_by: str) -> tuple[torch.T
 def _native_csr(rows: torch.Tensor, cols: torch.Tensor, num_nodes: int, want_order: bool):
     """(crow, col, order) from the native build, or Nones where it does not
     apply (see ``_native.csr_build_supported``)."""
-    if not rows.is_cuda:
+    if not rows.is_cuda or torch.compiler.is_compiling():
         return None, None, None
     from .. import _native
     from ..ops import load_native

@@ -116,6 +116,8 @@ def test_what_keeps_the_torch_composition():
     traced = make_fx(lambda e: edge_index_to_csr(e, 3))(torch.tensor([[0, 1, 2], [2, 2, 0]], device="cuda"))
     other = torch.tensor([[1, 0, 2], [0, 1, 0]], device="cuda")
     assert all(torch.equal(t, e) for t, e in zip(traced(other), edge_index_to_csr(other, 3)))
+    compiled = torch.compile(lambda e: edge_index_to_csr(e, 3), backend="eager", fullgraph=True)
+    assert all(torch.equal(t, e) for t, e in zip(compiled(other), edge_index_to_csr(other, 3)))
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         captured = _native.csr_build_supported(ids, ids, 3)
