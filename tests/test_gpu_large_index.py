@@ -122,6 +122,19 @@ def test_rounded_sddmm_past_32_bit_offsets(graph, dtype):
     del q, k
 
 
+@pytest.mark.parametrize("op", ["sddmm_csr", "sddmm_csr_rows"])
+def test_fp32_sddmm_past_32_bit_offsets(graph, op):
+    """Blocks of edges, and rows with hub rows in chunks."""
+    d_crow = torch.from_numpy(graph["crow"]).cuda()
+    d_col = torch.from_numpy(graph["col"]).cuda()
+    q = _device_values(N, F, torch.float32)
+    k = q.flip(1).contiguous()
+    want = oracle.sddmm_ref(graph["sub_crow"], graph["sub_col"], _values(graph["rows"], F),
+                            _values(graph["uniq"], F)[:, ::-1].copy())
+    assert np.array_equal(getattr(torch.ops.autosage, op)(d_crow, d_col, q, k).cpu().numpy(), want)
+    del q, k
+
+
 N_WIDE = (1 << 25) + 1000
 
 
